@@ -651,6 +651,20 @@ typedef struct SoupkLayerBwd {
 int soupk_layer_fwd(const SoupkLayerDims* dims, const SoupkLayerFwd* a, void* stream);
 int soupk_layer_bwd(const SoupkLayerDims* dims, const SoupkLayerBwd* a, void* stream);
 
+/*
+ * out [M, N] fp16 = a [M, K] @ b [K, N], fp16 row-major (leading dimensions lda, ldb, ldo in
+ * elements), for few output tiles and a long contraction: K is cut into parts whose fp32 partial
+ * products are added in a fixed order and rounded once.  The head's hidden gradient of up to some
+ * hundred labelled rows (solution/head.py:113).  N, K, lda, ldb multiples of 8, ldo of 4; a and b
+ * 16-byte, out 8-byte aligned; each operand under 2^30 elements.  `workspace`: 16-byte aligned,
+ * at least the floats soupk_gemm_nn_workspace gives for these sizes on the current device (0: NULL
+ * is fine).
+ */
+int soupk_gemm_nn(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, uint16_t* out,
+                  int64_t ldo, int64_t M, int32_t N, int32_t K, float* workspace,
+                  int64_t workspace_floats, void* stream);
+int soupk_gemm_nn_workspace(int64_t M, int32_t N, int32_t K, int64_t* floats);
+
 #ifdef __cplusplus
 }
 #endif

@@ -20,6 +20,7 @@ Operands outside these layouts go to torch (the same library, its own per-call s
 """
 
 import csv
+import ctypes
 import threading
 
 import torch
@@ -120,6 +121,38 @@ def matmul(a, b, bias=None, out=None, accumulate=False):
     _ext.call("soupk_gemm_lt", ta, 0, N, M, K, b.data_ptr(), lda, 0, a.data_ptr(), ldb, 0,
               out.data_ptr(), ldd, 0, 0, 1, 1 if accumulate else 0, _ext.ptr(bias),
               _table.get(key, -1), ws.data_ptr(), WORKSPACE_BYTES, st)
+    return out
+
+
+def _nn_workspace(M, N, K):
+    floats = ctypes.c_int64()
+    _ext.call("soupk_gemm_nn_workspace", M, N, K, ctypes.addressof(floats))
+    return floats.value
+
+
+def gemm_nn_fits(a, b, out):
+    """Operands soupk_gemm_nn takes: fp16 row-major on one device, 16-byte aligned rows, sizes in
+    multiples of 8, each under 2^30 elements."""
+    (M, K), N = a.shape, b.shape[1]
+    return (_fits(a) and _fits(b) and _fits(out) and a.device == b.device == out.device
+            and b.shape[0] == K and tuple(out.shape) == (M, N) and M > 0 and K > 0 and N > 0
+            and a.stride(1) == b.stride(1) == out.stride(1) == 1
+            and a.stride(0) >= K and b.stride(0) >= N and out.stride(0) >= N
+            and (K | N | a.stride(0) | b.stride(0) | out.stride(0)) % 8 == 0
+            and M * a.stride(0) < 1 << 30 and K * b.stride(0) < 1 << 30
+            and _aligned(a, b, out))
+
+
+def gemm_nn(a, b, out):
+    """out [M, N] = a [M, K] @ b [K, N] through soupk_gemm_nn (this package's split-K kernel: a few
+    hundred rows contracted over a very long K), each row-major with unit column stride."""
+    M, K = a.shape
+    N = b.shape[1]
+    floats = _nn_workspace(M, N, K)
+    ws = torch.empty(floats, dtype=torch.float32, device=a.device)
+    _ext.call("soupk_gemm_nn", a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+              out.data_ptr(), out.stride(0), M, N, K, ws.data_ptr() if floats else None, floats,
+              _ext.stream_of(a))
     return out
 
 

@@ -9,7 +9,8 @@ Design.  The rows (real tokens) are taken in their own order, CHUNK_ROWS at a ti
    stored straight at the row's place in the outputs, and for a labelled row the gradient
    (softmax - onehot) * scale in fp16, written to the row's slot in a buffer that holds only the
    chunk's labelled rows (the slot comes from a row map, -1 for an ignored row);
-3. hipBLASLt: dh = that buffer @ W, appended to one packed [labelled, H] gradient.
+3. testt_amd/csrc/gemm_nn.hip: dh = that buffer @ W, the contraction over the vocabulary cut into
+   parts that fill the chip, appended to one packed [labelled, H] gradient.
 The row map and the per-chunk labelled counts come from one cumulative sum over the labels and
 one host synchronisation (the counts size the dh GEMMs).  No row is ever permuted: the hidden
 states are read in place, the statistics need no unsort, and the backward forms the [M, H]
@@ -30,6 +31,7 @@ import math
 import torch
 
 from . import _ext
+from . import blas as _blas
 
 CHUNK_ROWS = 2048
 # Vocabulary tile of the reference's Triton loop (solution/head.py:30); the HIP kernel streams
@@ -104,6 +106,18 @@ def head_stats_grad_rows(logits, targets, grad_row, grad_out, entropy, token_los
                   _ext.ptr(grad_row), _ext.ptr(grad_out), n_out, _ext.ptr(entropy),
                   _ext.ptr(token_loss), _ext.ptr(correct), _ext.ptr(lse), float(grad_scale),
                   rows, vocab, _ext.stream_of(logits))
+
+
+def _hidden_grad(g, weight, out):
+    """out [n, H] = g [n, V] @ weight [V, H]: the split-K kernel for this shape (blas.gemm_nn: the
+    output is a few tiles and the contraction the whole vocabulary, which leaves a library GEMM
+    on part of the chip; 18 rows 326 -> 92 us, 420 rows 580 -> 249 us, 1536 rows 935 -> 686 us on
+    MI355X at 151936 x 1536, never slower from 1 to 2048 rows), hipBLASLt for operands it does
+    not take."""
+    if _blas.gemm_nn_fits(g, weight, out):
+        _blas.gemm_nn(g, weight, out)
+    else:
+        torch.matmul(g, weight, out=out)
 
 
 class _RowPlan:
@@ -188,7 +202,7 @@ class FusedHeadLoss(torch.autograd.Function):
             del logits
             if n_lab:
                 first = plan.lab_before[c]
-                torch.matmul(g, weight, out=packed[first:first + n_lab])
+                _hidden_grad(g, weight, packed[first:first + n_lab])
             del g
         total = token_loss.sum()
         loss = total / (denominator.to(dev) if torch.is_tensor(denominator) else denominator)
