@@ -652,17 +652,47 @@ int soupk_layer_fwd(const SoupkLayerDims* dims, const SoupkLayerFwd* a, void* st
 int soupk_layer_bwd(const SoupkLayerDims* dims, const SoupkLayerBwd* a, void* stream);
 
 /*
+ * The steps around the head's chunk kernels without a host synchronisation (replaces the sort, the
+ * count read-back and the scaled scatter of solution/head.py:93-137).
+ *
+ * soupk_head_plan: rows in chunks of `chunk`; slot[r] is row r's index among the labelled rows
+ * (target != -100) of its chunk, -1 for an ignored row; counts[c] the labelled rows of chunk c;
+ * scal[0] the gradient scale and scal[1] its unit: `scale` and `unit`, or, with a denominator in
+ * device memory, unit = the power of two nearest 64 * max(d, 1e-6) clamped to [1, 2^16] and
+ * scale = unit / max(d, 1e-6).
+ * soupk_head_stats_grad_planned: soupk_head_stats_grad_rows with the scale read from device memory.
+ * soupk_head_finish: loss[0] = sum(token_loss) / (denominator[0], or `den` when NULL), hit[r] =
+ * correct[r] != 0 as a byte.
+ * soupk_head_dh: dh [rows, H] fp16, dh[r] = fp16(packed[first row of r's chunk + slot[r]] *
+ * (grad_loss[0] / scal[1])), zeros where slot[r] is -1.
+ */
+int soupk_head_plan(const int64_t* target, int64_t rows, int64_t chunk, int32_t* slot,
+                    int32_t* counts, const int64_t* denominator, float scale, float unit,
+                    float* scal, void* stream);
+int soupk_head_stats_grad_planned(const uint16_t* logits, const int64_t* target,
+                                  const int32_t* grad_row, uint16_t* grad_out, int64_t grad_rows,
+                                  float* entropy, float* loss, int32_t* correct,
+                                  const float* grad_scale, int64_t rows, int64_t V, void* stream);
+int soupk_head_finish(const float* token_loss, const int32_t* correct, int64_t rows,
+                      const int64_t* denominator, float den, float* loss, uint8_t* hit,
+                      void* stream);
+int soupk_head_dh(const uint16_t* packed, const int32_t* slot, const float* grad_loss,
+                  const float* scal, uint16_t* dh, int64_t rows, int32_t H, int64_t chunk,
+                  void* stream);
+
+/*
  * out [M, N] fp16 = a [M, K] @ b [K, N], fp16 row-major (leading dimensions lda, ldb, ldo in
  * elements), for few output tiles and a long contraction: K is cut into parts whose fp32 partial
  * products are added in a fixed order and rounded once.  The head's hidden gradient of up to some
  * hundred labelled rows (solution/head.py:113).  N, K, lda, ldb multiples of 8, ldo of 4; a and b
- * 16-byte, out 8-byte aligned; each operand under 2^30 elements.  `workspace`: 16-byte aligned,
- * at least the floats soupk_gemm_nn_workspace gives for these sizes on the current device (0: NULL
- * is fine).
+ * 16-byte, out 8-byte aligned; each operand under 2^30 elements.  `rows`: NULL, or in device memory
+ * the number of leading rows of a that count (clamped to [0, M]); the rows of out past it are not
+ * written.  `workspace`: 16-byte aligned, at least the floats soupk_gemm_nn_workspace gives for
+ * these sizes on the current device.
  */
 int soupk_gemm_nn(const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, uint16_t* out,
-                  int64_t ldo, int64_t M, int32_t N, int32_t K, float* workspace,
-                  int64_t workspace_floats, void* stream);
+                  int64_t ldo, int64_t M, int32_t N, int32_t K, const int32_t* rows,
+                  float* workspace, int64_t workspace_floats, void* stream);
 int soupk_gemm_nn_workspace(int64_t M, int32_t N, int32_t K, int64_t* floats);
 
 #ifdef __cplusplus

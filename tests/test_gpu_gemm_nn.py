@@ -42,6 +42,23 @@ def test_gemm_nn(M, K, N):
     assert torch.equal(again.view(torch.int16), out.contiguous().view(torch.int16))
 
 
+@pytest.mark.parametrize("M,count", [(1, 0), (64, 33), (65, 1), (200, 200), (700, 420), (700, -1),
+                                     (300, 5000)])
+def test_gemm_nn_device_rows(M, count):
+    """The first `count` rows (clamped to [0, M]) computed, the others not written."""
+    K, N = 2056, 264
+    g = torch.Generator().manual_seed(M + count)
+    a = (0.05 * torch.randn(M, K, generator=g)).to(torch.float16).to(DEV)
+    b = (0.05 * torch.randn(K, N, generator=g)).to(torch.float16).to(DEV)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device=DEV)
+    n = min(max(count, 0), M)
+    a[n:] = float("inf")
+    blas.gemm_nn(a, b, out, torch.tensor([count], dtype=torch.int32, device=DEV))
+    assert bool(torch.isnan(out[n:]).all())
+    if n:
+        within_bound(out[:n], a[:n], b)
+
+
 def test_gemm_nn_refuses():
     a = torch.zeros(4, 16, dtype=torch.float16, device=DEV)
     b = torch.zeros(16, 8, dtype=torch.float16, device=DEV)

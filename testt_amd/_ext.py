@@ -44,6 +44,10 @@ SIGNATURES = {
     "soupk_swiglu_bwd_inplace": [_p, _p, _i64, _i64, _p],
     "soupk_head_stats_grad": [_p, _p, _p, _p, _p, _p, _f32, _i64, _i64, _p],
     "soupk_head_stats_grad_rows": [_p, _p, _p, _p, _i64, _p, _p, _p, _p, _f32, _i64, _i64, _p],
+    "soupk_head_plan": [_p, _i64, _i64, _p, _p, _p, _f32, _f32, _p, _p],
+    "soupk_head_stats_grad_planned": [_p, _p, _p, _p, _i64, _p, _p, _p, _p, _i64, _i64, _p],
+    "soupk_head_finish": [_p, _p, _i64, _p, _f32, _p, _p, _p],
+    "soupk_head_dh": [_p, _p, _p, _p, _p, _i64, _i32, _i64, _p],
     "soupk_time_next_launch": [_p, _p],
     "soupk_bench_copy": [_p, _p, _i64, _p],
     "soupk_bench_empty": [_i32, _p],
@@ -80,7 +84,7 @@ SIGNATURES = {
                       _i32, _i32, _i32, _p, _i32, _p, _i64, _p],
     "soupk_gemm_lt_index": [_i32, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                             _i32, _i32, _i32, _i32, _i32, _i64],
-    "soupk_gemm_nn": [_p, _i64, _p, _i64, _p, _i64, _i64, _i32, _i32, _p, _i64, _p],
+    "soupk_gemm_nn": [_p, _i64, _p, _i64, _p, _i64, _i64, _i32, _i32, _p, _p, _i64, _p],
     "soupk_gemm_nn_workspace": [_i64, _i32, _i32, _p],
     "soupk_layer_fwd": [_p, _p, _p],
     "soupk_layer_bwd": [_p, _p, _p],

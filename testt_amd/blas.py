@@ -143,15 +143,16 @@ def gemm_nn_fits(a, b, out):
             and _aligned(a, b, out))
 
 
-def gemm_nn(a, b, out):
+def gemm_nn(a, b, out, rows=None):
     """out [M, N] = a [M, K] @ b [K, N] through soupk_gemm_nn (this package's split-K kernel: a few
-    hundred rows contracted over a very long K), each row-major with unit column stride."""
+    hundred rows contracted over a very long K), each row-major with unit column stride.  `rows`:
+    int32 device tensor, the leading rows of a that count (the others are not written)."""
     M, K = a.shape
     N = b.shape[1]
     floats = _nn_workspace(M, N, K)
     ws = torch.empty(floats, dtype=torch.float32, device=a.device)
     _ext.call("soupk_gemm_nn", a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
-              out.data_ptr(), out.stride(0), M, N, K, ws.data_ptr() if floats else None, floats,
+              out.data_ptr(), out.stride(0), M, N, K, _ext.ptr(rows), ws.data_ptr(), floats,
               _ext.stream_of(a))
     return out
 

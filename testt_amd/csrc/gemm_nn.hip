@@ -52,24 +52,101 @@ __device__ __forceinline__ int xcd_local(int id, int total8) {
   return (id & 7) * (total8 >> 3) + (id >> 3);
 }
 
+struct NnPlan {
+  int tiles_m, tiles_n, splits, per;
+};
+
+// Most rows the 16- to 64-row tiles take; their two workgroups per CU.
+constexpr int kSmallRows = 64;
+
+// The row tile and the K parts.  The parts fill the CUs once (twice up to 64 rows, where two
+// workgroups fit a CU's LDS); a kernel plans them itself, from the rows that count.  Up to 192 rows one row of tiles, of the fewest rows that cover M;
+// above, the tile of 160, 192 or 256 rows with the least work per workgroup (rows x steps: the
+// three run at the same rate, 0.91 - 0.94 PFLOP/s where they are full; with 256-row tiles alone 640
+// rows took 369 us against 336, 1300 rows 681 against 598).  Two steps of prefetch instead of one
+// took the 160- and 192-row tiles from 147 and 152 us to 113 and 124 at one row of tiles; the
+// 256-row tile has no registers for the second.  The tile is the host's choice from the most rows;
+// the parts follow from the rows that count (420 of 700: 279 us on the tile for 700, 257 on the
+// tile for 420).
+__host__ __device__ inline NnPlan nn_plan(int bm, int M, int N, int K, int cus) {
+  NnPlan p;
+  p.tiles_m = (M + bm - 1) / bm;
+  p.tiles_n = (N + kNnBN - 1) / kNnBN;
+  const int kt = (K + kNnBK - 1) / kNnBK;
+  int s = cus * (bm <= kSmallRows ? 2 : 1) / (p.tiles_m * p.tiles_n);
+  s = s < 1 ? 1 : (s > kNnMaxSplits ? kNnMaxSplits : s);
+  s = s > kt ? kt : s;
+  p.per = (kt + s - 1) / s;
+  p.splits = (kt + p.per - 1) / p.per;
+  return p;
+}
+
+// The row tile for up to M rows.
+int nn_tile_rows(int M, int N, int K, int cus) {
+  if (M <= kSmallRows) return (M + 15) / 16 * 16;
+  if (M <= 192) return M <= 96 ? 96 : (M + 31) / 32 * 32;
+  int best = 256;
+  int64_t best_work = -1;
+  for (int bm : {256, 192, 160}) {
+    const NnPlan p = nn_plan(bm, M, N, K, cus);
+    const int wgs = p.tiles_m * p.tiles_n * p.splits;
+    const int64_t work = static_cast<int64_t>((wgs + cus - 1) / cus) * p.per * bm;
+    if (best_work < 0 || work < best_work) {
+      best = bm;
+      best_work = work;
+    }
+  }
+  return best;
+}
+
+struct NnArgs {
+  const uint16_t* a;
+  const uint16_t* b;
+  float* part;
+  uint16_t* out;
+  int64_t ldo;
+  uint32_t lda, ldb;
+  int M, N, K, cus;
+  const int32_t* rows;   // nullable: the rows of a that count (at most M), in device memory
+};
+
+__device__ __forceinline__ int nn_rows(const NnArgs& g) {
+  // (wave-uniform, and told so: the plan made of it stays in scalar registers)
+  return g.rows != nullptr ? __builtin_amdgcn_readfirstlane(max(0, min(*g.rows, g.M))) : g.M;
+}
+
 template <int MT, int WM, int PF>
-__global__ __launch_bounds__(kNnThreads, MT * WM <= 4 ? 4 : 2) void gemm_nn_kernel(
-    const uint16_t* a, uint32_t lda, const uint16_t* b, uint32_t ldb, float* __restrict__ part,
-    uint16_t* __restrict__ out, int64_t ldo, int M, int N, int K, int tiles_m, int tiles_n,
-    int splits, int per) {
+__global__ __launch_bounds__(kNnThreads, 16 * MT * WM <= kSmallRows ? 4 : 2) void gemm_nn_kernel(
+    NnArgs g) {
   constexpr int BM = 16 * MT * WM, WN = 8 / WM, NT = kNnBN / WN / 16;
   constexpr int AI = (BM + 63) / 64;          // 64-row groups of a's tile
-  constexpr int kABytes = BM * kNnBK * 2, kBBytes = kNnBK * kNnBN * 2;
-  __shared__ __align__(16) unsigned char smem[2][kABytes + kBBytes];
-  const int logical = xcd_local(blockIdx.x, gridDim.x);
-  const int tiles = tiles_m * tiles_n;
-  const int split = logical / tiles;
-  if (split >= splits) return;
+  constexpr int kABytes = BM * kNnBK * 2, kStage = kABytes + kNnBK * kNnBN * 2;
+  __shared__ __align__(16) unsigned char smem[2 * kStage];
+  // The plan is made from the row count in device memory (or M), so that a caller need not know the
+  // count; workgroups past the plan's exit.
+  const int M = nn_rows(g);
+  if (M == 0) return;
+  NnPlan p = nn_plan(BM, M, g.N, g.K, g.cus);
+  p.tiles_m = __builtin_amdgcn_readfirstlane(p.tiles_m);
+  p.tiles_n = __builtin_amdgcn_readfirstlane(p.tiles_n);
+  p.splits = __builtin_amdgcn_readfirstlane(p.splits);
+  p.per = __builtin_amdgcn_readfirstlane(p.per);
+  const int total = p.tiles_m * p.tiles_n * p.splits;
+  const int total8 = (total + 7) & ~7;
+  if (static_cast<int>(blockIdx.x) >= total8) return;
+  const int logical = xcd_local(blockIdx.x, total8);
+  if (logical >= total) return;
+  const uint16_t* const a = g.a;
+  const uint16_t* const b = g.b;
+  const uint32_t lda = g.lda, ldb = g.ldb;
+  const int N = g.N, K = g.K, splits = p.splits;
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int split = __builtin_amdgcn_readfirstlane(logical / tiles);
   const int tile = logical - split * tiles;
-  const int tm = tile % tiles_m, tn = tile / tiles_m;
+  const int tn = __builtin_amdgcn_readfirstlane(tile / p.tiles_m), tm = tile - tn * p.tiles_m;
   const int m0 = tm * BM, n0 = tn * kNnBN;
   const int kt = (K + kNnBK - 1) / kNnBK;
-  const int t0 = split * per, steps = min(per, kt - t0);
+  const int t0 = split * p.per, steps = min(p.per, kt - t0);
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w / WN, wn = w % WN;
@@ -109,7 +186,7 @@ __global__ __launch_bounds__(kNnThreads, MT * WM <= 4 ? 4 : 2) void gemm_nn_kern
       r.bv[i] = buf_load(rb, live ? boff + bt + static_cast<uint32_t>(i) * 32u * ldb : kOob);
   };
   auto store = [&](const Regs& r, int buf) {
-    unsigned char* sa = smem[buf];
+    unsigned char* sa = smem + buf * kStage;
     unsigned char* sb = sa + kABytes;
 #pragma unroll
     for (int i = 0; i < AI; ++i)
@@ -133,8 +210,8 @@ __global__ __launch_bounds__(kNnThreads, MT * WM <= 4 ? 4 : 2) void gemm_nn_kern
   const int brow = 8 * gr + (kk >> 2);
   const uint32_t b_sw = 2 * ((brow & 3) | (((brow >> 3) & 1) << 2));
   auto compute = [&](int buf) {
-    const unsigned char* sa = smem[buf];
-    const lds_b* sb = (const lds_b*)(smem[buf] + kABytes);
+    const unsigned char* sa = smem + buf * kStage;
+    const lds_b* sb = (const lds_b*)(sa + kABytes);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       // (the tallest tiles' registers hold one half step's fragments: no reads ahead of it)
@@ -172,12 +249,12 @@ __global__ __launch_bounds__(kNnThreads, MT * WM <= 4 ? 4 : 2) void gemm_nn_kern
     store(regs[(P + 1) % PF], P ^ 1);
     __syncthreads();
   };
-  int t = 0;
-  for (; t + 2 <= steps; t += 2) {
+  // (an odd last step is followed by one on zeros: a tail of its own made the compiler copy the
+  // accumulators every iteration)
+  for (int t = 0; t < steps; t += 2) {
     step(t, std::integral_constant<int, 0>{});
     step(t + 1, std::integral_constant<int, 1>{});
   }
-  if (t < steps) compute(0);
 
   // C: column (lane) = row of out, rows = columns 16j + 4gr .. +3 of the tile
 #pragma unroll
@@ -190,20 +267,25 @@ __global__ __launch_bounds__(kNnThreads, MT * WM <= 4 ? 4 : 2) void gemm_nn_kern
       if (n >= N) continue;
       const f32x4 v = acc[i][j];
       if (splits > 1)
-        *reinterpret_cast<f32x4*>(part + (static_cast<int64_t>(split) * M + m) * N + n) = v;
+        *reinterpret_cast<f32x4*>(g.part + (static_cast<int64_t>(split) * M + m) * N + n) = v;
       else
-        *reinterpret_cast<u32x2*>(out + m * ldo + n) =
+        *reinterpret_cast<u32x2*>(g.out + m * g.ldo + n) =
             u32x2{pack_h2(v[0], v[1]), pack_h2(v[2], v[3])};
     }
   }
 }
 
-// out = fp16_rn of the sum of the splits' partials: a workgroup takes 64 float4 columns-of-row,
-// wavefront w adds a quarter of the splits in order, the quarters are added in order.
-__global__ __launch_bounds__(256) void gemm_nn_sum_kernel(const f32x4* __restrict__ parts,
-                                                          int splits, int64_t n4, int n_cols4,
-                                                          uint16_t* __restrict__ out, int64_t ldo) {
+// out = fp16_rn of the sum of the parts: a workgroup takes 64 float4 columns-of-row, wavefront w
+// adds a quarter of the parts in order, the quarters are added in order.
+__global__ __launch_bounds__(256) void gemm_nn_sum_kernel(NnArgs g, int bm) {
   __shared__ f32x4 sums[3][64];
+  const int M = nn_rows(g);
+  const int n_cols4 = g.N / 4;
+  const int64_t n4 = static_cast<int64_t>(M) * n_cols4;
+  if (static_cast<int64_t>(blockIdx.x) * 64 >= n4) return;
+  const int splits = nn_plan(bm, M, g.N, g.K, g.cus).splits;
+  if (splits == 1) return;
+  const f32x4* const parts = reinterpret_cast<const f32x4*>(g.part);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + lane;
   const int64_t ic = min(i, n4 - 1);
@@ -224,51 +306,24 @@ __global__ __launch_bounds__(256) void gemm_nn_sum_kernel(const f32x4* __restric
   s = ((s + sums[0][lane]) + sums[1][lane]) + sums[2][lane];
   const int64_t m = i / n_cols4;
   const int64_t n = (i - m * n_cols4) * 4;
-  *reinterpret_cast<u32x2*>(out + m * ldo + n) = u32x2{pack_h2(s[0], s[1]), pack_h2(s[2], s[3])};
+  *reinterpret_cast<u32x2*>(g.out + m * g.ldo + n) =
+      u32x2{pack_h2(s[0], s[1]), pack_h2(s[2], s[3])};
 }
 
-struct NnPlan {
-  int bm, tiles_m, tiles_n, splits, per;
-};
+// Workgroups that any row count up to M can need: the CUs filled once (twice), or one part of
+// the most tiles.
+int64_t nn_grid(int bm, int64_t M, int32_t N, int cus) {
+  const int64_t tiles = (M + bm - 1) / bm * ((N + kNnBN - 1) / kNnBN);
+  return std::max<int64_t>(bm <= kSmallRows ? 2 * cus : cus, tiles);
+}
 
-// The row tile and the K parts.  The parts fill the CUs once (twice up to 64 rows, where two
-// workgroups fit a CU's LDS).  Up to 192 rows one row of tiles, of the fewest rows that cover M;
-// above, the tile of 160, 192 or 256 rows with the least work per workgroup (rows x steps: the
-// three run at the same rate, 0.91 - 0.94 PFLOP/s where they are full; with 256-row tiles alone 640
-// rows took 369 us against 336, 1300 rows 681 against 598).  Two steps of prefetch instead of one
-// took the 160- and 192-row tiles from 147 and 152 us to 113 and 124 at one row of tiles; the
-// 256-row tile has no registers for the second.
-NnPlan nn_plan(int64_t M, int32_t N, int32_t K) {
-  const int tiles_n = (N + kNnBN - 1) / kNnBN;
-  const int kt = (K + kNnBK - 1) / kNnBK;
-  const int cus = device_cu_count();
-  auto plan = [&](int bm) {
-    NnPlan p;
-    p.bm = bm;
-    p.tiles_m = static_cast<int>((M + bm - 1) / bm);
-    p.tiles_n = tiles_n;
-    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * tiles_n;
-    const int64_t fill = std::max<int64_t>(1, cus * (bm <= 64 ? 2 : 1) / tiles);
-    const int s = static_cast<int>(std::min<int64_t>(fill, std::min(kNnMaxSplits, kt)));
-    p.per = (kt + s - 1) / s;
-    p.splits = (kt + p.per - 1) / p.per;
-    return p;
-  };
-  const int rows = static_cast<int>(std::min<int64_t>(M, 1 << 20));
-  if (rows <= 64) return plan((rows + 15) / 16 * 16);
-  if (rows <= 192) return plan((rows + 31) / 32 * 32);
-  NnPlan best = plan(256);
-  int64_t best_work = -1;
-  for (int bm : {256, 192, 160}) {
-    const NnPlan p = plan(bm);
-    const int64_t wgs = static_cast<int64_t>(p.tiles_m) * tiles_n * p.splits;
-    const int64_t work = (wgs + cus - 1) / cus * p.per * bm;
-    if (best_work < 0 || work < best_work) {
-      best = p;
-      best_work = work;
-    }
-  }
-  return best;
+// Floats of the partials for any row count up to M: with more than one part, tiles x parts fill
+// the CUs at most once (twice), so the parts' rows x columns are at most that many whole tiles.
+int64_t nn_workspace(int64_t M, int32_t N, int32_t K, int cus) {
+  const bool small = M <= kSmallRows;
+  const int64_t kt = (K + kNnBK - 1) / kNnBK;
+  const int64_t tiles = static_cast<int64_t>(small ? 2 * cus * kSmallRows : cus * 256) * kNnBN;
+  return std::min(tiles, std::min<int64_t>(kNnMaxSplits, kt) * M * N);
 }
 
 int check_nn(const void* a, int64_t lda, const void* b, int64_t ldb, const void* out, int64_t ldo,
@@ -293,34 +348,33 @@ using namespace soupk;
 extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_workspace(
     int64_t M, int32_t N, int32_t K, int64_t* floats) {
   if (M < 0 || N <= 0 || K <= 0 || !floats || M > (1 << 20)) return kInvalid;
-  *floats = 0;
-  if (M == 0) return kOk;
-  const NnPlan p = nn_plan(M, N, K);
-  if (p.splits > 1) *floats = static_cast<int64_t>(p.splits) * M * N;
+  *floats = nn_workspace(M, N, K, device_cu_count());
   return kOk;
 }
 
 extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn(
     const uint16_t* a, int64_t lda, const uint16_t* b, int64_t ldb, uint16_t* out, int64_t ldo,
-    int64_t M, int32_t N, int32_t K, float* workspace, int64_t workspace_floats, void* stream) {
+    int64_t M, int32_t N, int32_t K, const int32_t* rows, float* workspace,
+    int64_t workspace_floats, void* stream) {
   const int rc0 = check_nn(a, lda, b, ldb, out, ldo, M, N, K);
   if (rc0 != kOk) return rc0;
   if (M == 0) return kOk;
-  const NnPlan p = nn_plan(M, N, K);
-  const int64_t need = p.splits > 1 ? static_cast<int64_t>(p.splits) * M * N : 0;
-  if (need > 0 && (!workspace || workspace_floats < need ||
-                   (reinterpret_cast<uintptr_t>(workspace) & 15)))
+  const int cus = device_cu_count();
+  if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
+      workspace_floats < nn_workspace(M, N, K, cus))
     return kInvalid;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int total = p.tiles_m * p.tiles_n * p.splits;
-  const dim3 grid(static_cast<unsigned>((total + 7) / 8 * 8)), block(kNnThreads);
+  const int bm = nn_tile_rows(static_cast<int>(M), N, K, cus);
+  const int64_t wgs = (nn_grid(bm, M, N, cus) + 7) / 8 * 8;
+  const int64_t sums = (M * N / 4 + 63) / 64;
+  if (wgs > 0x7fffffff || sums > 0x7fffffff) return kInvalid;
+  const NnArgs g{a, b, workspace, out, ldo, static_cast<uint32_t>(lda), static_cast<uint32_t>(ldb),
+                 static_cast<int>(M), N, K, cus, rows};
   auto run = [&](auto kernel) {
-    return launch_kernel(kernel, grid, block, st, a, static_cast<uint32_t>(lda), b,
-                         static_cast<uint32_t>(ldb), workspace, out, ldo, static_cast<int>(M), N, K,
-                         p.tiles_m, p.tiles_n, p.splits, p.per);
+    return launch_kernel(kernel, dim3(static_cast<unsigned>(wgs)), dim3(kNnThreads), st, g);
   };
   int rc;
-  switch (p.bm) {
+  switch (bm) {
     case 16: rc = run(gemm_nn_kernel<1, 1, 2>); break;
     case 32: rc = run(gemm_nn_kernel<2, 1, 2>); break;
     case 48: rc = run(gemm_nn_kernel<3, 1, 2>); break;
@@ -329,11 +383,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn(
     case 128: rc = run(gemm_nn_kernel<4, 2, 2>); break;
     case 160: rc = run(gemm_nn_kernel<5, 2, 2>); break;
     case 192: rc = run(gemm_nn_kernel<6, 2, 2>); break;
-    case 256: rc = run(gemm_nn_kernel<8, 2, 1>); break;
-    default: return kInvalid;
+    default: rc = run(gemm_nn_kernel<8, 2, 1>); break;
   }
-  if (rc != kOk || p.splits == 1) return rc;
-  const int64_t n4 = M * N / 4;
-  return launch_kernel(gemm_nn_sum_kernel, dim3(static_cast<unsigned>((n4 + 63) / 64)), dim3(256),
-                       st, reinterpret_cast<const f32x4*>(workspace), p.splits, n4, N / 4, out, ldo);
+  // (one part whatever the row count: the tiles alone fill the CUs, or K is one step)
+  if (rc != kOk ||
+      (rows == nullptr && nn_plan(bm, static_cast<int>(M), N, K, cus).splits == 1))
+    return rc;
+  return launch_kernel(gemm_nn_sum_kernel, dim3(static_cast<unsigned>(sums)), dim3(256), st, g, bm);
 }

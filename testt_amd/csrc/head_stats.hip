@@ -238,6 +238,7 @@ struct GradDest {
   uint16_t* grad_out;       // nullable
   int64_t grad_rows;
   bool in_place;
+  const float* scale;       // nullable: the gradient scale in device memory (soupk_head_plan's)
 };
 
 __device__ __forceinline__ uint16_t* grad_row_base(const GradDest& gd, uint16_t* base,
@@ -399,6 +400,7 @@ __global__ __launch_bounds__(kHeadThreads) void head_stats_grad_kernel(
                                loss, correct, lse_out, kLift);
   uint16_t* const gbase = grad_row_base(gd, base, row, V);
   if (!labelled || gbase == nullptr) return;
+  if (gd.scale != nullptr) grad_scale = *gd.scale;
   // The gradient row has the logits row's alignment (the entry point checks it), so it splits
   // into the same lead columns, whole chunks and tail columns.
   const __amdgpu_buffer_rsrc_t wrsrc =
@@ -481,6 +483,7 @@ __global__ __launch_bounds__(kHeadThreads) void head_stats_grad_stream_kernel(
                                loss, correct, lse_out, 0.f);
   uint16_t* const gbase = grad_row_base(gd, base, row, V);
   if (!labelled || gbase == nullptr) return;
+  if (gd.scale != nullptr) grad_scale = *gd.scale;
   u32x4* const gvb = reinterpret_cast<u32x4*>(gbase + sp.lead);
   const float shift = -lse * kLog2e;
   const int64_t tc = (tgt_ok && tgt >= sp.lead && tgt < sp.tail0) ? (tgt - sp.lead) >> 3 : -1;
@@ -510,6 +513,16 @@ __global__ __launch_bounds__(kHeadThreads) void head_stats_grad_stream_kernel(
 using namespace soupk;
 
 namespace {
+
+// Every gradient row must split into the same lead columns, 16-byte chunks and tail columns as
+// every logits row: the same address modulo 16 and a row pitch of whole chunks.
+bool bad_grad_rows(const uint16_t* logits, const int32_t* grad_row, const uint16_t* grad_out,
+                   int64_t grad_rows, int64_t V) {
+  if ((grad_out == nullptr) != (grad_row == nullptr) || grad_rows < 0) return true;
+  return grad_out != nullptr &&
+         ((V * 2) % 16 != 0 ||
+          ((reinterpret_cast<uintptr_t>(grad_out) - reinterpret_cast<uintptr_t>(logits)) & 15u));
+}
 
 int head_launch(uint16_t* logits, const int64_t* target, float* entropy, float* loss,
                 int32_t* correct, float* lse_out, float grad_scale, int64_t rows, int64_t V,
@@ -546,7 +559,7 @@ int head_launch(uint16_t* logits, const int64_t* target, float* entropy, float* 
 extern "C" __attribute__((visibility("default"))) int soupk_head_stats_grad(
     uint16_t* logits, const int64_t* target, float* entropy, float* loss, int32_t* correct,
     float* lse_out, float grad_scale, int64_t rows, int64_t V, void* stream) {
-  const GradDest gd{nullptr, nullptr, 0, true};
+  const GradDest gd{nullptr, nullptr, 0, true, nullptr};
   return head_launch(logits, target, entropy, loss, correct, lse_out, grad_scale, rows, V, gd,
                      stream);
 }
@@ -555,16 +568,20 @@ extern "C" __attribute__((visibility("default"))) int soupk_head_stats_grad_rows
     const uint16_t* logits, const int64_t* target, const int32_t* grad_row, uint16_t* grad_out,
     int64_t grad_rows, float* entropy, float* loss, int32_t* correct, float* lse_out,
     float grad_scale, int64_t rows, int64_t V, void* stream) {
-  if ((grad_out == nullptr) != (grad_row == nullptr) || grad_rows < 0) return kInvalid;
-  if (grad_out != nullptr) {
-    // Every gradient row must split into the same lead columns, 16-byte chunks and tail
-    // columns as every logits row: the same address modulo 16 and a row pitch of whole chunks.
-    if ((V * 2) % 16 != 0) return kInvalid;
-    if ((reinterpret_cast<uintptr_t>(grad_out) - reinterpret_cast<uintptr_t>(logits)) & 15u)
-      return kInvalid;
-  }
-  const GradDest gd{grad_row, grad_out, grad_rows, false};
+  if (bad_grad_rows(logits, grad_row, grad_out, grad_rows, V)) return kInvalid;
+  const GradDest gd{grad_row, grad_out, grad_rows, false, nullptr};
   // The kernels only read the logits when the gradient goes elsewhere (or nowhere).
   return head_launch(const_cast<uint16_t*>(logits), target, entropy, loss, correct, lse_out,
                      grad_scale, rows, V, gd, stream);
+}
+
+extern "C" __attribute__((visibility("default"))) int soupk_head_stats_grad_planned(
+    const uint16_t* logits, const int64_t* target, const int32_t* grad_row, uint16_t* grad_out,
+    int64_t grad_rows, float* entropy, float* loss, int32_t* correct, const float* grad_scale,
+    int64_t rows, int64_t V, void* stream) {
+  if (bad_grad_rows(logits, grad_row, grad_out, grad_rows, V)) return kInvalid;
+  if (rows > 0 && grad_out != nullptr && !grad_scale) return kInvalid;
+  const GradDest gd{grad_row, grad_out, grad_rows, false, grad_scale};
+  return head_launch(const_cast<uint16_t*>(logits), target, entropy, loss, correct, nullptr, 0.f,
+                     rows, V, gd, stream);
 }

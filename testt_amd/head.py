@@ -11,12 +11,13 @@ Design.  The rows (real tokens) are taken in their own order, CHUNK_ROWS at a ti
    chunk's labelled rows (the slot comes from a row map, -1 for an ignored row);
 3. testt_amd/csrc/gemm_nn.hip: dh = that buffer @ W, the contraction over the vocabulary cut into
    parts that fill the chip, appended to one packed [labelled, H] gradient.
-The row map and the per-chunk labelled counts come from one cumulative sum over the labels and
-one host synchronisation (the counts size the dh GEMMs).  No row is ever permuted: the hidden
-states are read in place, the statistics need no unsort, and the backward forms the [M, H]
-gradient in one gather from the packed rows (an appended zero row serves the ignored ones),
-scaled by the loss scale on the way.  The gradient is taken in the forward because the head is
-frozen.
+The row map, the per-chunk labelled counts and the gradient's scale stay on the device
+(testt_amd/csrc/head_plan.hip; the dh kernel reads the count it covers), so the whole head is
+enqueued without waiting for the GPU; a vocabulary or denominator this form does not take keeps
+a row plan read back to the host (_RowPlan).  No row is ever permuted: the hidden states are read
+in place, the statistics need no unsort, and the backward forms the [M, H] gradient in one gather
+from the packed rows, scaled by the loss scale on the way.  The gradient is taken in the forward
+because the head is frozen.
 
 CHUNK_ROWS keeps the reference's name; its value is MI355X's: the reference's 256 rows bound
 the logits buffer on a 15 GB card (78 MB), while 2048 rows (622 MB, plus the labelled rows'
@@ -154,6 +155,85 @@ class _RowPlan:
         self.gather = torch.where(labelled, (seen - 1).to(torch.int64), self.n_labelled)
 
 
+def _denominator_args(denominator, device):
+    """(device pointer or None, host value, kept tensor) of a denominator the device plan takes: a
+    Python number, or an integer tensor of no dimensions on `device`; None for any other."""
+    if torch.is_tensor(denominator):
+        if denominator.device != device or denominator.dim() != 0 or \
+                denominator.dtype not in (torch.int64, torch.int32):
+            return None
+        den = denominator.to(torch.int64)
+        return den.data_ptr(), 0.0, den
+    if isinstance(denominator, (int, float)):
+        return None, float(denominator), None
+    return None
+
+
+def _device_plan(hidden, weight, denominator):
+    """The arguments of the forward without a host synchronisation, or None where the general
+    form runs: fp16 rows and head on one device, a vocabulary whose rows are whole 16-byte chunks
+    (the gradient rows keep the logits rows' alignment) and operands gemm_nn takes."""
+    rows, width = hidden.shape
+    vocab = weight.shape[0]
+    if rows == 0 or not hidden.is_cuda or hidden.dtype != torch.float16 or \
+            weight.dtype != torch.float16 or weight.device != hidden.device or \
+            not weight.is_contiguous() or weight.dim() != 2 or weight.shape[1] != width or \
+            vocab % 8 or width % 8 or weight.data_ptr() % 16 or vocab * width >= 1 << 30 or \
+            min(rows, CHUNK_ROWS) * vocab >= 1 << 30:
+        return None
+    return _denominator_args(denominator, hidden.device)
+
+
+def _forward_device(ctx, hidden, weight, targets, den):
+    """FusedHeadLoss.forward with the row plan, the scale and the labelled counts on the device."""
+    den_ptr, den_host, den_keep = den
+    rows, width = hidden.shape
+    vocab = weight.shape[0]
+    dev = hidden.device
+    st = _ext.stream_of(hidden)
+    chunk = CHUNK_ROWS
+    entropy = torch.empty(rows, dtype=torch.float32, device=dev)
+    token_loss = torch.empty(rows, dtype=torch.float32, device=dev)
+    correct = torch.empty(rows, dtype=torch.int32, device=dev)
+    want_grad = ctx.needs_input_grad[0]
+    slot = packed = scal = None
+    if want_grad:
+        unit = _grad_unit(den_host) if den_ptr is None else 0.0
+        scale = unit / max(den_host, 1e-6)
+        slot = torch.empty(rows, dtype=torch.int32, device=dev)
+        counts = torch.empty(-(-rows // chunk), dtype=torch.int32, device=dev)
+        scal = torch.empty(2, dtype=torch.float32, device=dev)
+        packed = torch.empty((rows, width), dtype=torch.float16, device=dev)
+        _ext.call("soupk_head_plan", targets.data_ptr(), rows, chunk, slot.data_ptr(),
+                  counts.data_ptr(), den_ptr, scale, unit, scal.data_ptr(), st)
+    for c, start in enumerate(range(0, rows, chunk)):
+        stop = min(rows, start + chunk)
+        n = stop - start
+        logits = torch.matmul(hidden[start:stop], weight.t())
+        g = torch.empty((n, vocab), dtype=torch.float16, device=dev) if want_grad else None
+        _ext.call("soupk_head_stats_grad_planned", logits.data_ptr(),
+                  targets.data_ptr() + 8 * start,
+                  slot.data_ptr() + 4 * start if want_grad else None, _ext.ptr(g),
+                  n if want_grad else 0, entropy.data_ptr() + 4 * start,
+                  token_loss.data_ptr() + 4 * start, correct.data_ptr() + 4 * start,
+                  _ext.ptr(scal), n, vocab, st)
+        del logits
+        if want_grad:
+            _blas.gemm_nn(g, weight, packed[start:stop], counts[c:c + 1])
+        del g
+    loss = torch.empty((), dtype=torch.float32, device=dev)
+    hit = torch.empty(rows, dtype=torch.bool, device=dev)
+    _ext.call("soupk_head_finish", token_loss.data_ptr(), correct.data_ptr(), rows, den_ptr,
+              den_host, loss.data_ptr(), hit.data_ptr(), st)
+    ctx.planned = want_grad
+    if want_grad:
+        ctx.chunk = chunk
+        ctx.save_for_backward(packed, slot, scal)
+    stats = (entropy, token_loss, hit)
+    ctx.mark_non_differentiable(*stats)
+    return (loss, *stats)
+
+
 class FusedHeadLoss(torch.autograd.Function):
     """(loss, entropy [M], token loss [M], correct [M]) of the frozen head over `hidden`
     (solution/head.py:87-137's interface); the gradient for `hidden` is computed in forward."""
@@ -164,6 +244,10 @@ class FusedHeadLoss(torch.autograd.Function):
         vocab = weight.shape[0]
         dev = hidden.device
         targets = targets.to(torch.int64).contiguous()
+        den = _device_plan(hidden, weight, denominator)
+        if den is not None and targets.device == dev and targets.numel() == rows:
+            return _forward_device(ctx, hidden.contiguous(), weight, targets, den)
+        ctx.planned = False
         entropy = torch.empty(rows, dtype=torch.float32, device=dev)
         token_loss = torch.empty(rows, dtype=torch.float32, device=dev)
         correct = torch.empty(rows, dtype=torch.int32, device=dev)
@@ -217,6 +301,14 @@ class FusedHeadLoss(torch.autograd.Function):
     def backward(ctx, grad_loss, *_unused):
         if not ctx.needs_input_grad[0]:
             return None, None, None, None
+        if ctx.planned:
+            packed, slot, scal = ctx.saved_tensors
+            grad_loss = grad_loss.to(torch.float32).contiguous()
+            dh = torch.empty_like(packed)
+            _ext.call("soupk_head_dh", packed.data_ptr(), slot.data_ptr(), grad_loss.data_ptr(),
+                      scal.data_ptr(), dh.data_ptr(), packed.shape[0], packed.shape[1], ctx.chunk,
+                      _ext.stream_of(dh))
+            return dh, None, None, None
         packed, gather = ctx.saved_tensors
         factor = grad_loss.to(torch.float32) / ctx.unit
         if gather is None:
