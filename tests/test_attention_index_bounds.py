@@ -79,6 +79,26 @@ def replay(cu, M, NH, NKV, T_rope=None):
                 if st.any():
                     assert ((base + q_abs[st]) * HD + h * D + 16 * 7 + 4 * gr[st] + 3).max() < out_n
                     assert (h * M + base + q_abs[st]).max() < lse_n
+            # the 128-query forward: z -> query block nw - 1 - z, wavefront w its 32 queries
+            nw = -(-length // 128)
+            for z in range(-(-M // 128)):
+                qb = nw - 1 - z
+                if qb < 0:
+                    continue
+                n_kb = min(2 * qb + 2, -(-length // BK))
+                for u in range(2):
+                    q_abs = qb * 128 + 32 * w + 16 * u + ql
+                    qrow = np.minimum(q_abs, length - 1)
+                    assert ((base + qrow) * W + h * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
+                    st = q_abs < length
+                    # a stored query's own key block is among those staged
+                    assert (q_abs[st] // BK < n_kb).all()
+                    if st.any():
+                        assert ((base + q_abs[st]) * HD + h * D + 16 * 7 + 4 * gr[st] + 3).max() \
+                            < out_n
+                for kb in range(n_kb + 1):
+                    _check_tile(kb * BK, length, base, W, (NH + g) * D, qkv_n)
+                    _check_tile(kb * BK, length, base, W, (NH + NKV + g) * D, qkv_n)
             # backward: even z -> dK/dV of key block z/2, odd z -> dQ of query block nb-1-z/2
             for z in range(2 * slots):
                 if z % 2 == 0:

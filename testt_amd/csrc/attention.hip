@@ -34,6 +34,7 @@
 
 #include "fastdiv.hpp"
 #include "soupk_common.hpp"
+#include <type_traits>
 
 namespace soupk {
 namespace {
@@ -278,6 +279,60 @@ __device__ __forceinline__ SeqHead seq_head(const AttnParams& p, int b, int h) {
   return s;
 }
 
+// The online softmax of one block for one 16-query tile: sc holds this lane's 16 raw scores
+// (-inf: masked), pb gets their probabilities 2^(s * scale_log2 - m_ref) in the order of the two
+// C-tile pairs.  A query's reference value m_ref is raised to the block's maximum when that
+// exceeds it by more than the margin, a decision of that query alone (its accumulators are then
+// rescaled by alpha, and by exactly 1 for the others of the wavefront), so that the result of a
+// query does not depend on which queries share its wavefront: the 64- and the 128-query kernels
+// give the same bits.
+//
+// (`maximum`, gfx950's three-operand NaN-propagating form: fmaxf first quiets every operand, one
+// more instruction per score.  A NaN score makes its query's sums NaN either way.)
+template <int U>
+__device__ __forceinline__ void softmax_block(const f4 (&sc)[U][4], float scale_log2,
+                                              float (&m_ref)[U], float (&lsum)[U],
+                                              f4 (&acc)[U][8], h8 (&pb)[U][2]) {
+  float m_new[U];
+  bool raise[U], any = false;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float mx = sc[u][0][0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = __builtin_elementwise_maximum(mx, sc[u][e >> 2][e & 3]);
+    mx = column_max(mx) * scale_log2;
+    raise[u] = mx > m_ref[u] + kRescaleMargin;   // (m_ref = -inf: any visible key)
+    m_new[u] = raise[u] ? mx : m_ref[u];
+    any = any | raise[u];
+  }
+  if (__any(any)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float alpha = raise[u] ? __builtin_amdgcn_exp2f(m_ref[u] - m_new[u]) : 1.f;  // 2^-inf = 0
+      lsum[u] *= alpha;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) acc[u][t] = acc[u][t] * alpha;
+      m_ref[u] = m_new[u];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float m_use = m_ref[u] == -INFINITY ? 0.f : m_ref[u];
+    float ps = 0.f;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float pr = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(sc[u][n][i], scale_log2, -m_use));  // 2^-inf = 0
+        ps += pr;
+        pb[u][n >> 1][4 * (n & 1) + i] = static_cast<_Float16>(pr);
+      }
+    }
+    lsum[u] += ps;
+  }
+}
+
 // One query block of one (sequence, head): flash-attention forward.
 __device__ __forceinline__ void attn_fwd_block(const AttnParams& p, const SeqHead& sh, int qb,
                                                _Float16* Ks, _Float16* Vs, uint8_t* kflag) {
@@ -296,10 +351,10 @@ __device__ __forceinline__ void attn_fwd_block(const AttnParams& p, const SeqHea
   h8 qf[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) qf[s] = *reinterpret_cast<const h8*>(qrow + 32 * s + 8 * gr);
-  f4 acc[8];
+  f4 acc[1][8];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  float m_ref = -INFINITY, lsum = 0.f;
+  for (int t = 0; t < 8; ++t) acc[0][t] = f4{0.f, 0.f, 0.f, 0.f};
+  float m_ref[1] = {-INFINITY}, lsum[1] = {0.f};
 
   TileRegs kr, vr;
   load_tile(kr, kbase, sh.ld_kv, 0, T);
@@ -320,7 +375,7 @@ __device__ __forceinline__ void attn_fwd_block(const AttnParams& p, const SeqHea
     // flight instead of one keep the MFMA pipe busy; pinned with scheduling-group barriers,
     // since the compiler otherwise reads each fragment just before its use and runs one tile's
     // chain after another: 15.52 -> 15.22 us at 2048 tokens, 12.83 -> 12.21 us ragged).
-    f4 sc[4];
+    f4 sc[1][4];
     {
       h8 kf[4][4];
 #pragma unroll
@@ -329,18 +384,16 @@ __device__ __forceinline__ void attn_fwd_block(const AttnParams& p, const SeqHea
         for (int s = 0; s < 4; ++s)
           kf[n][s] = lds_h8(Ks + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
 #pragma unroll
-      for (int n = 0; n < 4; ++n) sc[n] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int n = 0; n < 4; ++n) sc[0][n] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int n = 0; n < 4; ++n) sc[n] = mfma32(kf[n][s], qf[s], sc[n]);
+        for (int n = 0; n < 4; ++n) sc[0][n] = mfma32(kf[n][s], qf[s], sc[0][n]);
       __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);   // the 16 LDS reads
       __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);   // then the 16 MFMAs
     }
-    // scale, mask (the diagonal block, or keys with flags), block max.  Keys of an interior
-    // block (kb < qb) precede every query of this workgroup and lie below T.
-    float x[4][4];
-    float mx = -INFINITY;
+    // mask (the diagonal block, or keys with flags), then the softmax of the block.  Keys of an
+    // interior block (kb < qb) precede every query of this workgroup and lie below T.
     if (kb == qb || has_valid) {
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
@@ -349,61 +402,31 @@ __device__ __forceinline__ void attn_fwd_block(const AttnParams& p, const SeqHea
         for (int i = 0; i < 4; ++i) {
           const int key = kb * kBK + 16 * n + 4 * gr + i;
           const bool vis = key <= q_abs && ((fl >> (8 * i)) & 0xffu) != 0;
-          x[n][i] = vis ? sc[n][i] * scale_log2 : -INFINITY;
-          mx = fmaxf(mx, x[n][i]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          x[n][i] = sc[n][i] * scale_log2;
-          mx = fmaxf(mx, x[n][i]);
+          sc[0][n][i] = vis ? sc[0][n][i] : -INFINITY;
         }
       }
     }
-    mx = column_max(mx);
-    if (__any(mx > m_ref + kRescaleMargin)) {   // (m_ref = -inf: any visible key)
-      const float m_new = fmaxf(m_ref, mx);
-      const float alpha = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
-      lsum *= alpha;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) acc[t] = acc[t] * alpha;
-      m_ref = m_new;
-    }
-    const float m_use = m_ref == -INFINITY ? 0.f : m_ref;
-    float ps = 0.f;
-    h8 pb[2];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float pr = __builtin_amdgcn_exp2f(x[n][i] - m_use);  // 2^-inf = 0
-        ps += pr;
-        pb[n >> 1][4 * (n & 1) + i] = static_cast<_Float16>(pr);
-      }
-    }
-    lsum += ps;
+    h8 pb[1][2];
+    softmax_block<1>(sc, scale_log2, m_ref, lsum, acc, pb);
     // O^T += V^T P^T
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
 #pragma unroll
       for (int m = 0; m < 2; ++m)
-        acc[t] = mfma32(lds_runs_tr(Vs, kRStride, 16 * t, m, gr), pb[m], acc[t]);
+        acc[0][t] = mfma32(lds_runs_tr(Vs, kRStride, 16 * t, m, gr), pb[0][m], acc[0][t]);
     }
   }
-  const float l_tot = column_sum(lsum);
+  const float l_tot = column_sum(lsum[0]);
   if (q_abs >= T) return;
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   uint16_t* orow = sh.out + static_cast<uint32_t>(q_abs) * static_cast<uint32_t>(sh.ld_o);
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
-    const f4 o = acc[t] * inv;
+    const f4 o = acc[0][t] * inv;
     *reinterpret_cast<u32x2*>(orow + 16 * t + 4 * gr) = u32x2{pack_h2(o[0], o[1]),
                                                                 pack_h2(o[2], o[3])};
   }
-  if (gr == 0) sh.lse[q_abs] = l_tot > 0.f ? (m_ref + log2f(l_tot)) * kLn2 : INFINITY;
+  if (gr == 0) sh.lse[q_abs] = l_tot > 0.f ? (m_ref[0] + log2f(l_tot)) * kLn2 : INFINITY;
 }
 
 // Grid: x = head, y = sequence (batch row), z = query-block slot: slot z is query block
@@ -428,6 +451,134 @@ __global__ __launch_bounds__(kAttnThreads) void attn_fwd_kernel(AttnParams p) {
   const SeqHead sh = seq_head<VARLEN>(p, blockIdx.y, blockIdx.x);
   const int qb = (sh.len + kBQ - 1) / kBQ - 1 - static_cast<int>(blockIdx.z);
   if (qb >= 0) attn_fwd_block(p, sh, qb, Ks, Vs, kflag);
+}
+
+// ---- forward of long sequences: 128 queries per workgroup ------------------------------------
+// A wavefront owns 32 queries (two 16-query tiles), so every K and V fragment it reads from LDS
+// serves two products instead of one: at 16 queries per wavefront the LDS reads of a block take as
+// long as its MFMAs (each 1024 clocks per CU), here half as long.  The next block's tiles go from
+// registers into the other of two LDS buffers, one barrier per block, and two workgroups fit a
+// CU (73.9 KB of LDS, two wavefronts per SIMD), so one's softmax runs under the other's MFMAs.
+// 2 x 4096 tokens, 12 heads: 222 -> 141 us (464 -> 733 TFLOP/s).  What is left is the chain of a
+// block (scores, maxima, exponentials, products) at two wavefronts per SIMD.  A workgroup order that
+// gives each XCD's L2 its own heads measured nothing on even rows and 129 -> 251 us on rows of 4096
+// to 1024 tokens (the XCDs' shares differ); raising the wave priority around the MFMAs 150 -> 157 us.
+constexpr int kWideBQ = 128;
+
+template <bool VARLEN>
+__global__ __launch_bounds__(kAttnThreads, 2) void attn_fwd_wide_kernel(AttnParams p) {
+  __shared__ __align__(16) _Float16 Ks[2][kBK * kRStride];
+  __shared__ __align__(16) _Float16 Vs[2][kBK * kRStride];
+  __shared__ __align__(16) uint8_t kflag[2][kBK];
+  const SeqHead sh = seq_head<VARLEN>(p, blockIdx.y, blockIdx.x);
+  const int T = sh.len;
+  const int qb = (T + kWideBQ - 1) / kWideBQ - 1 - static_cast<int>(blockIdx.z);
+  if (qb < 0) return;
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const int ql = lane & 15, gr = lane >> 4;
+  const int q0 = qb * kWideBQ + 32 * w;              // this wavefront's first query
+  const int n_kb = min(2 * qb + 2, (T + kBK - 1) / kBK);
+  const int kb_diag = q0 / kBK;                      // the block of its queries' own keys
+  const bool has_valid = sh.valid != nullptr;
+  const float scale_log2 = p.scale_log2;
+  h8 qf[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const uint16_t* qrow = row_at(sh.q, min(q0 + 16 * u + ql, T - 1), sh.ld_q);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) qf[u][s] = *reinterpret_cast<const h8*>(qrow + 32 * s + 8 * gr);
+  }
+  f4 acc[2][8];
+  float m_ref[2] = {-INFINITY, -INFINITY}, lsum[2] = {0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[u][t] = f4{0.f, 0.f, 0.f, 0.f};
+
+  TileRegs kr, vr;
+  uint8_t fl_raw = 0;
+  auto load = [&](int kb) {
+    load_tile(kr, sh.k, sh.ld_kv, kb * kBK, T);
+    load_tile(vr, sh.v, sh.ld_kv, kb * kBK, T);
+    if (has_valid) fl_raw = load_flag_raw(sh.valid, sh.k, kb * kBK, T);
+  };
+  auto store = [&](int kb) {
+    store_tile(Ks[kb & 1], kr);
+    store_tile(Vs[kb & 1], vr);
+    if (has_valid && threadIdx.x < kBK)
+      kflag[kb & 1][threadIdx.x] = key_flag(fl_raw, true, kb * kBK, T);
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  // One key block for this wavefront's two query tiles; MASK: the block of the queries' own keys,
+  // or keys with flags.
+  auto block = [&](int kb, auto mask) {
+    const _Float16* K = Ks[kb & 1];
+    const _Float16* V = Vs[kb & 1];
+    f4 sc[2][4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      h8 kf[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) kf[s] = lds_h8(K + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
+      sc[0][n] = sc[1][n] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sc[u][n] = mfma32(kf[s], qf[u][s], sc[u][n]);
+    }
+    if constexpr (decltype(mask)::value) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const uint32_t fl = has_valid ? flag_word(kflag[kb & 1], n, gr) : 0x01010101u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = kb * kBK + 16 * n + 4 * gr + i;
+          const bool real = ((fl >> (8 * i)) & 0xffu) != 0;
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            sc[u][n][i] = (key <= q0 + 16 * u + ql && real) ? sc[u][n][i] : -INFINITY;
+        }
+      }
+    }
+    h8 pb[2][2];
+    softmax_block<2>(sc, scale_log2, m_ref, lsum, acc, pb);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const h8 vf = lds_runs_tr(V, kRStride, 16 * t, m, gr);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) acc[u][t] = mfma32(vf, pb[u][m], acc[u][t]);
+      }
+    }
+  };
+  for (int kb = 0; kb < n_kb; ++kb) {
+    load(kb + 1);      // (clamped past the end)
+    issue_here();
+    if (kb < kb_diag && (VARLEN || !has_valid))
+      block(kb, std::false_type{});
+    else if (kb <= kb_diag)
+      block(kb, std::true_type{});
+    store(kb + 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int q_abs = q0 + 16 * u + ql;
+    const float l_tot = column_sum(lsum[u]);
+    if (q_abs >= T) continue;
+    const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+    uint16_t* orow = sh.out + static_cast<uint32_t>(q_abs) * static_cast<uint32_t>(sh.ld_o);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const f4 o = acc[u][t] * inv;
+      *reinterpret_cast<u32x2*>(orow + 16 * t + 4 * gr) = u32x2{pack_h2(o[0], o[1]),
+                                                                  pack_h2(o[2], o[3])};
+    }
+    if (gr == 0) sh.lse[q_abs] = l_tot > 0.f ? (m_ref[u] + log2f(l_tot)) * kLn2 : INFINITY;
+  }
 }
 
 // ---- backward ------------------------------------------------------------------------------
@@ -900,6 +1051,16 @@ int check_varlen(int32_t B, int64_t M, int32_t NH, int32_t NKV, int32_t D, float
   return kOk;
 }
 
+// Whether the 128-query forward takes `units` (sequence, head) pairs of `len` rows on average:
+// where its workgroups are at least 5/4 of the CUs.  Below, the 64-query kernel's shorter chains
+// fill the chip better.  Measured (us, 64 / 128 queries per workgroup, 12 heads): 2 x 4096 rows 222 /
+// 141, 1 x 4096 (384 workgroups) 124 / 116, 16 x 256 (384) 29.9 / 17.8, 4 x 1024 (384) 40.6 / 34.0,
+// 2 rows of 2500 and 800 (312) 76 / 75, 1 x 3000 (288) 75 / 82, 2 x 1365 (264) 36 / 42, 4 x 512 (192)
+// 15.4 / 20.5.
+bool wide_forward(int64_t units, int64_t len) {
+  return units * ((len + kWideBQ - 1) / kWideBQ) * 4 >= int64_t{5} * device_cu_count();
+}
+
 bool misaligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; }
 
 AttnParams base_params(int32_t NH, int32_t NKV, float scale) {
@@ -936,6 +1097,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_fwd(
   p.out = out;
   p.lse = lse;
   p.T = T;
+  if (wide_forward(static_cast<int64_t>(B) * NH, T))
+    return launch_kernel(attn_fwd_wide_kernel<false>,
+                         dim3(static_cast<unsigned>(NH), static_cast<unsigned>(B),
+                              static_cast<unsigned>((T + kWideBQ - 1) / kWideBQ)),
+                         dim3(kAttnThreads), static_cast<hipStream_t>(stream), p);
   const dim3 grid(static_cast<unsigned>(NH), static_cast<unsigned>(B),
                   static_cast<unsigned>((T + kBQ - 1) / kBQ));
   return launch_kernel(attn_fwd_kernel<false>, grid, dim3(kAttnThreads),
@@ -1006,6 +1172,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_varlen_fwd
   p.M = M;
   p.W = static_cast<int64_t>(NH + 2 * NKV) * kD;
   const int slots = static_cast<int>((M + kBQ - 1) / kBQ);
+  if (wide_forward(static_cast<int64_t>(B) * NH, M / B))   // (slots for a sequence of all M tokens)
+    return launch_kernel(attn_fwd_wide_kernel<true>,
+                         dim3(static_cast<unsigned>(NH), static_cast<unsigned>(B),
+                              static_cast<unsigned>((M + kWideBQ - 1) / kWideBQ)),
+                         dim3(kAttnThreads), static_cast<hipStream_t>(stream), p);
   const dim3 grid(static_cast<unsigned>(NH), static_cast<unsigned>(B),
                   static_cast<unsigned>(slots));
   return launch_kernel(attn_fwd_kernel<true>, grid, dim3(kAttnThreads),
