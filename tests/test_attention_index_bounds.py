@@ -1,8 +1,8 @@
 """CPU regression test: the varlen attention kernels' index arithmetic stays in bounds.
 
 testt_amd/csrc/attention.hip launches the varlen forward on a (heads, sequences, ceil(M/64))
-grid, the backward on (heads, sequences, 2 ceil(M/64)) (even z: dK/dV of a key block, odd z:
-dQ of a query block), the delta kernel on (heads, 1, ceil(M/64)) and the reduce on M*NKV*16
+grid, or of 128-query blocks on (heads, sequences, ceil(M/128)), the backward on (heads,
+sequences, 3 ceil(M/128)) (of three z, two dK/dV of a key block, one dQ of 128 queries), the delta kernel on (heads, 1, ceil(M/64)) and the reduce on M*NKV*16
 items.  Workgroups past a sequence's blocks exit; rows are clamped to the sequence's last row
 before every load; sequence bounds come from device memory (cu_seqlens) and a bound outside
 [0, M] empties the sequence.  This test replays that arithmetic with numpy for every workgroup
@@ -99,10 +99,12 @@ def replay(cu, M, NH, NKV, T_rope=None):
                 for kb in range(n_kb + 1):
                     _check_tile(kb * BK, length, base, W, (NH + g) * D, qkv_n)
                     _check_tile(kb * BK, length, base, W, (NH + NKV + g) * D, qkv_n)
-            # backward: even z -> dK/dV of key block z/2, odd z -> dQ of query block nb-1-z/2
-            for z in range(2 * slots):
-                if z % 2 == 0:
-                    kb = z // 2
+            # backward, z = 3 zq + zr: zr < 2 -> dK/dV of key block 2 zq + zr, zr = 2 -> dQ of
+            # 128-query block nw - 1 - zq
+            for z in range(3 * -(-M // 128)):
+                zq, zr = z // 3, z % 3
+                if zr < 2:
+                    kb = 2 * zq + zr
                     if kb >= nb:
                         continue
                     key = kb * BK + 16 * w + ql
@@ -117,26 +119,29 @@ def replay(cu, M, NH, NKV, T_rope=None):
                     if st.any():
                         assert ((h * M + base + key[st]) * D + 16 * 7 + 4 * gr[st] + 3).max() < part_n
                 else:
-                    qb = nb - 1 - z // 2
+                    qb = nw - 1 - zq
                     if qb < 0:
                         continue
-                    q_abs = qb * BQ + 16 * w + ql
-                    qc = np.minimum(q_abs, length - 1)
-                    assert ((base + qc) * W + h * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
-                    assert ((base + qc) * HD + h * D + 32 * 3 + 8 * gr + 7).max() < out_n
-                    assert (h * M + base + qc).max() < lse_n
-                    for kb in range(qb + 2):
+                    n_kb = min(2 * qb + 2, -(-length // BK))
+                    for u in range(2):
+                        q_abs = qb * 128 + 32 * w + 16 * u + ql
+                        qc = np.minimum(q_abs, length - 1)
+                        assert ((base + qc) * W + h * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
+                        assert ((base + qc) * HD + h * D + 32 * 3 + 8 * gr + 7).max() < out_n
+                        assert (h * M + base + qc).max() < lse_n
+                        st = q_abs < length
+                        assert (q_abs[st] // BK < n_kb).all()
+                        if st.any():
+                            tok = base + q_abs[st]
+                            assert tok.max() < M
+                            # dQ row, first and second half (RoPE's transposed rotation)
+                            assert (tok * W + h * D + 16 * 3 + 4 * gr[st] + 64 + 3).max() < qkv_n
+                            if T_rope is not None:
+                                # table row t < T_rope, dims d .. d+3 and d+64 .. d+67, d <= 60
+                                assert 60 + 64 + 3 < D
+                    for kb in range(n_kb + 1):
                         _check_tile(kb * BK, length, base, W, (NH + g) * D, qkv_n)
                         _check_tile(kb * BK, length, base, W, (NH + NKV + g) * D, qkv_n)
-                    st = q_abs < length
-                    if st.any():
-                        tok = base + q_abs[st]
-                        assert tok.max() < M
-                        # dQ row, first and second half (RoPE's transposed rotation)
-                        assert (tok * W + h * D + 16 * 3 + 4 * gr[st] + 64 + 3).max() < qkv_n
-                        if T_rope is not None:
-                            # table row t < T_rope, dims d .. d+3 and d+64 .. d+67, d <= 60
-                            assert 60 + 64 + 3 < D
     # delta: the padded kernel over one row of M positions (b = 0, T = M)
     for h in range(NH):
         for qb in range(slots):

@@ -63,6 +63,8 @@ def test_varlen_wide_matches_row_launches(lengths):
     cu = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32,
                       device=DEV)
     out, lse = attention.attention_varlen_fwd(rows, cu, NH, NKV, SCALE)
+    dout = (0.1 * torch.randn(M, NH * D, generator=g)).to(torch.float16).to(DEV)
+    dqkv = attention.attention_varlen_bwd(rows, cu, out, lse, dout, SCALE, NH, NKV)
     at = 0
     for n in lengths:
         if n:
@@ -72,4 +74,7 @@ def test_varlen_wide_matches_row_launches(lengths):
                                                     SCALE)
             assert torch.equal(o1.view(torch.int16), out[at:at + n].view(torch.int16)), n
             assert torch.equal(l1, lse[:, at:at + n]), n
+            d1 = attention.attention_varlen_bwd(rows[at:at + n].contiguous(), one, o1, l1,
+                                                dout[at:at + n], SCALE, NH, NKV)
+            assert torch.equal(d1.view(torch.int16), dqkv[at:at + n].view(torch.int16)), n
         at += n

@@ -587,9 +587,9 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_fwd_wide_kernel(AttnPara
 // dK = scale * dS^T Q,  dV = P^T dO.  Three launches:
 //   attn_bwd_delta_kernel (b, head, 64 queries): D;
 //   attn_bwd_kernel       two kinds of workgroup in one grid, so that they run side by side
-//                         (z even: dK/dV of 64 keys, z odd: dQ of 64 queries, the heaviest
+//                         (of three z, two dK/dV of 64 keys and one dQ of 128 queries, the heaviest
 //                         causal blocks of both kinds dispatched first):
-//     dQ   (b, head, 64 queries): over its key blocks S^T = K Q^T, dP^T = V dO^T (the
+//     dQ   (b, head, 128 queries): over its key blocks S^T = K Q^T, dP^T = V dO^T (the
 //          forward's orientation: query = lane column), dQ^T += K^T dS^T;
 //     dKdV (b, head, 64 keys): over the query blocks that see them, S = Q K^T, dP = dO V^T
 //          (key = lane column), dV^T += dO^T P, dK^T += Q^T dS, into fp32 partials per query
@@ -631,10 +631,6 @@ __global__ __launch_bounds__(kAttnThreads) void attn_bwd_delta_kernel(
   if (gr == 0 && q_abs < T) delta[(static_cast<int64_t>(b) * NH + h) * T + q_abs] = dsum;
 }
 
-// LDS of the backward workgroups (the larger of the two kinds: dKdV's Q and dO tiles and the
-// block's lse / D values).
-constexpr int kBwdLdsBytes = 2 * kBQ * kRStride * 2 + 2 * kBQ * 4;
-
 // fp32 -> fp16 -> fp32: the value a kernel that stores fp16 hands to the next one.
 __device__ __forceinline__ float round_h(float x) { return lo_h(pack_h2(x, 0.f)); }
 
@@ -672,85 +668,10 @@ __device__ __forceinline__ void rope_bwd4(const float* c, const float* sn, int d
   rope_bwd4(c1, c2, s1, s2, g1, g2, o1, o2);
 }
 
+// The dQ row of query q_abs from its accumulators (this lane: dims 16t + 4gr .. +3).
 template <bool VARLEN>
-__device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& sh, int h, int b,
-                                            int qb, unsigned char* smem) {
-  _Float16* Ks = reinterpret_cast<_Float16*>(smem);
-  _Float16* Vs = Ks + kBK * kRStride;
-  uint8_t* kflag = reinterpret_cast<uint8_t*>(Vs + kBK * kRStride);
-  const int T = sh.len;
-  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
-  const int ql = lane & 15, gr = lane >> 4;
-  const int q_abs = qb * kBQ + 16 * w + ql;
-  const int qc = min(q_abs, T - 1);
-  const uint16_t* qrow = row_at(sh.q, qc, sh.ld_q);
-  const uint16_t* dorow = row_at(sh.dout, qc, sh.ld_o);
-  const uint16_t* kbase = sh.k;
-  const uint16_t* vbase = sh.v;
-  const uint8_t* valid = sh.valid;
-  const bool has_valid = valid != nullptr;
-  const float scale_log2 = p.scale_log2;
-
-  h8 qf[4], dof[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    qf[s] = *reinterpret_cast<const h8*>(qrow + 32 * s + 8 * gr);
-    dof[s] = *reinterpret_cast<const h8*>(dorow + 32 * s + 8 * gr);
-  }
-  const float dsum = sh.delta[qc];
-  const float lse2 = sh.lse[qc] * kLog2e;  // +inf: no visible key, every p = 0
-
-  f4 acc[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-  TileRegs kr, vr;
-  load_tile(kr, kbase, sh.ld_kv, 0, T);
-  load_tile(vr, vbase, sh.ld_kv, 0, T);
-  uint8_t fl_raw = load_flag_raw(valid, kbase, 0, T);
-  for (int kb = 0; kb <= qb; ++kb) {
-    __syncthreads();
-    store_tile(Ks, kr);   // K^T fragments read transposed from Ks
-    store_tile(Vs, vr);
-    if (threadIdx.x < kBK) kflag[threadIdx.x] = key_flag(fl_raw, has_valid, kb * kBK, T);
-    __syncthreads();
-    load_tile(kr, kbase, sh.ld_kv, (kb + 1) * kBK, T);   // the next block (clamped past the end)
-    load_tile(vr, vbase, sh.ld_kv, (kb + 1) * kBK, T);
-    fl_raw = load_flag_raw(valid, kbase, (kb + 1) * kBK, T);
-    issue_here();
-    const bool masked = kb == qb || has_valid;
-    h8 dsb[2];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      h8 kf[4], vf[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        kf[s] = lds_h8(Ks + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
-        vf[s] = lds_h8(Vs + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
-      }
-      f4 sc = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        sc = mfma32(kf[s], qf[s], sc);
-        dp = mfma32(vf[s], dof[s], dp);
-      }
-      const uint32_t fl = masked ? flag_word(kflag, n, gr) : 0x01010101u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int key = kb * kBK + 16 * n + 4 * gr + i;
-        const bool vis = !masked || (key <= q_abs && ((fl >> (8 * i)) & 0xffu) != 0);
-        const float pr = vis ? __builtin_amdgcn_exp2f(sc[i] * scale_log2 - lse2) : 0.f;
-        dsb[n >> 1][4 * (n & 1) + i] = static_cast<_Float16>(pr * (dp[i] - dsum));
-      }
-    }
-    // dQ^T += K^T dS^T
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-#pragma unroll
-      for (int m = 0; m < 2; ++m)
-        acc[t] = mfma32(lds_runs_tr(Ks, kRStride, 16 * t, m, gr), dsb[m], acc[t]);
-    }
-  }
-  if (q_abs >= T) return;
+__device__ __forceinline__ void store_dq(const AttnParams& p, const SeqHead& sh, int h, int b,
+                                         int q_abs, int gr, const f4 (&acc)[8]) {
   const float scale = p.scale;
   if constexpr (VARLEN) {
     // dq|dk|dv row of the token; with tables, dQ is rounded to fp16 (the value an attention
@@ -799,12 +720,131 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& 
   }
 }
 
+// dQ of 128 queries: 32 per wavefront, so that every K and V fragment read from LDS serves two
+// tiles (at 16 the LDS reads of a block take as long as its MFMAs), double-buffered tiles with one
+// barrier per block, as the 128-query forward.
+template <bool VARLEN>
+__device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& sh, int h,
+                                                 int b, int qb, unsigned char* smem) {
+  const int T = sh.len;
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  const int ql = lane & 15, gr = lane >> 4;
+  const int q0 = qb * kWideBQ + 32 * w;
+  const int n_kb = min(2 * qb + 2, (T + kBK - 1) / kBK);
+  const int kb_diag = q0 / kBK;
+  const bool has_valid = sh.valid != nullptr;
+  const float scale_log2 = p.scale_log2;
+  constexpr int kTile = kBK * kRStride;               // halves
+  _Float16* const tiles = reinterpret_cast<_Float16*>(smem);    // K, V of buffer 0, then of 1
+  uint8_t* const flags = smem + 4 * kTile * 2;
+  h8 qf[2][4], dof[2][4];
+  float dsum[2], lse2[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int qc = min(q0 + 16 * u + ql, T - 1);
+    const uint16_t* qrow = row_at(sh.q, qc, sh.ld_q);
+    const uint16_t* dorow = row_at(sh.dout, qc, sh.ld_o);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      qf[u][s] = *reinterpret_cast<const h8*>(qrow + 32 * s + 8 * gr);
+      dof[u][s] = *reinterpret_cast<const h8*>(dorow + 32 * s + 8 * gr);
+    }
+    dsum[u] = sh.delta[qc];
+    lse2[u] = sh.lse[qc] * kLog2e;   // +inf: no visible key, every p = 0
+  }
+  f4 acc[2][8];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[u][t] = f4{0.f, 0.f, 0.f, 0.f};
+  TileRegs kr, vr;
+  uint8_t fl_raw = 0;
+  auto load = [&](int kb) {
+    load_tile(kr, sh.k, sh.ld_kv, kb * kBK, T);
+    load_tile(vr, sh.v, sh.ld_kv, kb * kBK, T);
+    if (!VARLEN && has_valid) fl_raw = load_flag_raw(sh.valid, sh.k, kb * kBK, T);
+  };
+  auto store = [&](int kb) {
+    store_tile(tiles + (kb & 1) * 2 * kTile, kr);
+    store_tile(tiles + ((kb & 1) * 2 + 1) * kTile, vr);
+    if (!VARLEN && has_valid && threadIdx.x < kBK)
+      flags[(kb & 1) * kBK + threadIdx.x] = key_flag(fl_raw, true, kb * kBK, T);
+  };
+  auto block = [&](int kb, auto mask) {
+    const _Float16* K = tiles + (kb & 1) * 2 * kTile;
+    const _Float16* V = K + kTile;
+    h8 dsb[2][2];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      h8 kf[4], vf[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        kf[s] = lds_h8(K + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
+        vf[s] = lds_h8(V + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
+      }
+      f4 sc[2], dp[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) sc[u] = dp[u] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          sc[u] = mfma32(kf[s], qf[u][s], sc[u]);
+          dp[u] = mfma32(vf[s], dof[u][s], dp[u]);
+        }
+      const uint32_t fl = !VARLEN && has_valid ? flag_word(flags + (kb & 1) * kBK, n, gr)
+                                               : 0x01010101u;
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = kb * kBK + 16 * n + 4 * gr + i;
+          float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[u][i], scale_log2, -lse2[u]));
+          if constexpr (decltype(mask)::value) {
+            const bool vis = (key <= q0 + 16 * u + ql) & (((fl >> (8 * i)) & 0xffu) != 0);
+            pr = vis ? pr : 0.f;
+          }
+          dsb[u][n >> 1][4 * (n & 1) + i] = static_cast<_Float16>(pr * (dp[u][i] - dsum[u]));
+        }
+    }
+    // dQ^T += K^T dS^T
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const h8 kt = lds_runs_tr(K, kRStride, 16 * t, m, gr);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) acc[u][t] = mfma32(kt, dsb[u][m], acc[u][t]);
+      }
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int kb = 0; kb < n_kb; ++kb) {
+    load(kb + 1);      // (clamped past the end)
+    issue_here();
+    if (kb < kb_diag && (VARLEN || !has_valid))
+      block(kb, std::false_type{});
+    else if (kb <= kb_diag)
+      block(kb, std::true_type{});
+    store(kb + 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int q_abs = q0 + 16 * u + ql;
+    if (q_abs < T) store_dq<VARLEN>(p, sh, h, b, q_abs, gr, acc[u]);
+  }
+}
+
+// dK/dV of 64 keys, 16 per wavefront (32 would take 128 accumulator and 64 operand registers: more
+// than two wavefronts per SIMD have), double-buffered tiles and one barrier per block.  Loading the
+// next 16 queries' fragments ahead of this tile's exponentials spills and doubles the time.
 __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead& sh, int kb,
-                                              unsigned char* smem) {
-  _Float16* Qs = reinterpret_cast<_Float16*>(smem);
-  _Float16* Ds = Qs + kBQ * kRStride;   // dO row-major
-  float* lse2_s = reinterpret_cast<float*>(Ds + kBQ * kRStride);
-  float* delta_s = lse2_s + kBQ;
+                                                   unsigned char* smem) {
+  constexpr int kTile = kBQ * kRStride;
+  _Float16* const tiles = reinterpret_cast<_Float16*>(smem);   // Q, dO of buffer 0, then of 1
+  float* const stats = reinterpret_cast<float*>(smem + 4 * kTile * 2);   // lse2, D of 0, of 1
   const int T = sh.len;
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int kl = lane & 15, gr = lane >> 4;
@@ -814,14 +854,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
   const bool has_valid = sh.valid != nullptr;
   const uint16_t* krow = row_at(sh.k, kc, sh.ld_kv);
   const uint16_t* vrow = row_at(sh.v, kc, sh.ld_kv);
-  const uint16_t* qbase = sh.q;
-  const uint16_t* dobase = sh.dout;
-  const float* lse_bh = sh.lse;
-  const float* del_bh = sh.delta;
   const float scale_log2 = p.scale_log2;
-
-  // K^T and V^T operands (B of S = Q K^T and of dP = dO V^T): lane holds row key of K / V,
-  // dims 32s + 8gr .. +7
   h8 kf[4], vf[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
@@ -833,38 +866,36 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
   for (int t = 0; t < 8; ++t) dk[t] = dv[t] = f4{0.f, 0.f, 0.f, 0.f};
   const int nqb = (T + kBQ - 1) / kBQ;
   TileRegs qr, dr;
-  float lse_raw, del_raw;   // tested against T only when stored (see load_flag_raw)
-  auto load_block = [&](int q0) {
-    load_tile(qr, qbase, sh.ld_q, q0, T);
-    load_tile(dr, dobase, sh.ld_o, q0, T);
-    const int t = min(q0 + (static_cast<int>(threadIdx.x) & (kBQ - 1)), T - 1);
-    lse_raw = lse_bh[t];
-    del_raw = del_bh[t];
+  float lse_raw, del_raw;
+  auto load = [&](int qb) {
+    load_tile(qr, sh.q, sh.ld_q, qb * kBQ, T);
+    load_tile(dr, sh.dout, sh.ld_o, qb * kBQ, T);
+    const int t = min(qb * kBQ + (static_cast<int>(threadIdx.x) & (kBQ - 1)), T - 1);
+    lse_raw = sh.lse[t];
+    del_raw = sh.delta[t];
   };
-  load_block(kb * kBQ);
-  for (int qb = kb; qb < nqb; ++qb) {
-    __syncthreads();
-    store_tile(Qs, qr);   // Q^T, dO^T fragments read transposed
-    store_tile(Ds, dr);
+  auto store = [&](int qb) {
+    const int bf = qb & 1;
+    store_tile(tiles + bf * 2 * kTile, qr);
+    store_tile(tiles + (bf * 2 + 1) * kTile, dr);
     if (threadIdx.x < kBQ) {
       const bool in = qb * kBQ + static_cast<int>(threadIdx.x) < T;
-      lse2_s[threadIdx.x] = in ? lse_raw * kLog2e : INFINITY;
-      delta_s[threadIdx.x] = in ? del_raw : 0.f;
+      stats[bf * 2 * kBQ + threadIdx.x] = in ? lse_raw * kLog2e : INFINITY;
+      stats[(bf * 2 + 1) * kBQ + threadIdx.x] = in ? del_raw : 0.f;
     }
-    __syncthreads();
-    load_block((qb + 1) * kBQ);   // the next block (clamped past the end)
-    issue_here();
-    // Every (query, key) pair of an interior block is visible: the queries follow the keys,
-    // lie below T, and no flags apply.
-    const bool masked = qb == kb || has_valid || (qb + 1) * kBQ > T;
+  };
+  auto block = [&](int qb, auto mask) {
+    const _Float16* Q = tiles + (qb & 1) * 2 * kTile;
+    const _Float16* O = Q + kTile;
+    const float* l2s = stats + (qb & 1) * 2 * kBQ;
     h8 pb[2], dsb[2];
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       h8 qa[4], da[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        qa[s] = lds_h8(Qs + (16 * n + kl) * kRStride + 32 * s + 8 * gr);
-        da[s] = lds_h8(Ds + (16 * n + kl) * kRStride + 32 * s + 8 * gr);
+        qa[s] = lds_h8(Q + (16 * n + kl) * kRStride + 32 * s + 8 * gr);
+        da[s] = lds_h8(O + (16 * n + kl) * kRStride + 32 * s + 8 * gr);
       }
       f4 sc = {0.f, 0.f, 0.f, 0.f}, dp = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -872,34 +903,41 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
         sc = mfma32(qa[s], kf[s], sc);
         dp = mfma32(da[s], vf[s], dp);
       }
-      // C: rows = queries 16n + 4gr + i, column = this lane's key.  The per-query values are
-      // read and every exponential computed unconditionally, the mask applied as a select:
-      // a conditional LDS read would put each of them behind its own branch and wait.
-      const f4 l2 = *reinterpret_cast<const f4*>(lse2_s + 16 * n + 4 * gr);
-      const f4 dl = *reinterpret_cast<const f4*>(delta_s + 16 * n + 4 * gr);
+      const f4 l2 = *reinterpret_cast<const f4*>(l2s + 16 * n + 4 * gr);
+      const f4 dl = *reinterpret_cast<const f4*>(l2s + kBQ + 16 * n + 4 * gr);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int q_abs = qb * kBQ + 16 * n + 4 * gr + i;
-        // (bitwise, not short-circuit: no per-lane branch)
-        const bool vis = !masked | (key_vis & (key_abs <= q_abs) & (q_abs < T));
-        const float e = __builtin_amdgcn_exp2f(sc[i] * scale_log2 - l2[i]);
-        const float pr = vis ? e : 0.f;
+        float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], scale_log2, -l2[i]));
+        if constexpr (decltype(mask)::value) {
+          const int q_abs = qb * kBQ + 16 * n + 4 * gr + i;
+          pr = (key_vis & (key_abs <= q_abs) & (q_abs < T)) ? pr : 0.f;
+        }
         pb[n >> 1][4 * (n & 1) + i] = static_cast<_Float16>(pr);
         dsb[n >> 1][4 * (n & 1) + i] = static_cast<_Float16>(pr * (dp[i] - dl[i]));
       }
     }
-    // dV^T += dO^T P, dK^T += Q^T dS  (contraction over the block's queries)
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
+    for (int t = 0; t < 8; ++t)
 #pragma unroll
       for (int m = 0; m < 2; ++m) {
-        dv[t] = mfma32(lds_runs_tr(Ds, kRStride, 16 * t, m, gr), pb[m], dv[t]);
-        dk[t] = mfma32(lds_runs_tr(Qs, kRStride, 16 * t, m, gr), dsb[m], dk[t]);
+        dv[t] = mfma32(lds_runs_tr(O, kRStride, 16 * t, m, gr), pb[m], dv[t]);
+        dk[t] = mfma32(lds_runs_tr(Q, kRStride, 16 * t, m, gr), dsb[m], dk[t]);
       }
-    }
+  };
+  load(kb);
+  store(kb);
+  __syncthreads();
+  for (int qb = kb; qb < nqb; ++qb) {
+    load(qb + 1);   // (clamped past the end)
+    issue_here();
+    if (qb == kb || has_valid || (qb + 1) * kBQ > T)
+      block(qb, std::true_type{});
+    else
+      block(qb, std::false_type{});
+    store(qb + 1);
+    __syncthreads();
   }
   if (key_abs >= T) return;
-  // C: rows = dims 16t + 4gr + i, column = this lane's key
   float* dkp = p.dk_part + (sh.plane + key_abs) * kD;
   float* dvp = p.dv_part + (sh.plane + key_abs) * kD;
   const float scale = p.scale;
@@ -910,19 +948,26 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
   }
 }
 
-// Grid z = 2 * slots (as the forward's): z even -> dKdV of key block z/2 (block 0 sees the
-// most query blocks), z odd -> dQ of query block nqb-1-z/2 (the last sees the most key blocks).
+constexpr int kBwdLdsBytes = 4 * kBK * kRStride * 2 + 4 * kBQ * 4;
+
+// Grid z = 3 * (128-query slots): z % 3 == 2 -> dQ of a 128-query block, the others dK/dV of 64 keys,
+// the heaviest causal blocks of both kinds first.  Against 64-query dQ workgroups and single LDS
+// tiles with two barriers a block (delta and reduce launches included, 12 heads, us): 2 x 4096 tokens
+// 537 -> 452, 1 x 8000 907 -> 814, rows of 4096 to 1024 477 -> 406, 4 x 1024 100 -> 94, 16 x 256 82 ->
+// 72, 4 x 512 42.2 -> 41.4, rows of 512 to 96 32.3 -> 32.5.  Bound by the dK/dV chain: 64 MFMAs, as
+// many clocks of LDS reads and 16 exponentials a block, at two wavefronts per SIMD.
 template <bool VARLEN>
-__global__ __launch_bounds__(kAttnThreads) void attn_bwd_kernel(AttnParams p) {
+__global__ __launch_bounds__(kAttnThreads, 2) void attn_bwd_kernel(AttnParams p) {
   __shared__ __align__(16) unsigned char smem[kBwdLdsBytes];
   const int h = blockIdx.x, b = blockIdx.y;
   const SeqHead sh = seq_head<VARLEN>(p, b, h);
-  const int nb = (sh.len + kBQ - 1) / kBQ;
-  const int z = static_cast<int>(blockIdx.z);
-  if ((z & 1) == 0) {
-    if ((z >> 1) < nb) attn_bwd_dkdv(p, sh, z >> 1, smem);
-  } else if (nb - 1 - (z >> 1) >= 0) {
-    attn_bwd_dq<VARLEN>(p, sh, h, b, nb - 1 - (z >> 1), smem);
+  const int z = static_cast<int>(blockIdx.z), zq = z / 3, zr = z - 3 * zq;
+  if (zr < 2) {
+    const int kb = 2 * zq + zr;
+    if (kb < (sh.len + kBK - 1) / kBK) attn_bwd_dkdv(p, sh, kb, smem);
+  } else {
+    const int qb = (sh.len + kWideBQ - 1) / kWideBQ - 1 - zq;
+    if (qb >= 0) attn_bwd_dq<VARLEN>(p, sh, h, b, qb, smem);
   }
 }
 
@@ -1042,7 +1087,7 @@ int check_shape(int32_t B, int32_t T, int32_t NH, int32_t NKV, int32_t D, float 
   return kOk;
 }
 
-// ... and by the varlen ones (the grid's z covers ceil(M/64) block slots, twice backward).
+// ... and by the varlen ones (the grid's z covers ceil(M/64) block slots; backward, three per 128).
 int check_varlen(int32_t B, int64_t M, int32_t NH, int32_t NKV, int32_t D, float scale) {
   if (B < 0 || M < 0 || NH <= 0 || NKV <= 0 || NH % NKV != 0 || D != kD) return kInvalid;
   if (!(scale > 0.f)) return kInvalid;
@@ -1148,7 +1193,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_bwd(
                          p.delta, T, NH);
   if (rc != kOk) return rc;
   const dim3 grid2(static_cast<unsigned>(NH), static_cast<unsigned>(B),
-                   static_cast<unsigned>(2 * nb));
+                   static_cast<unsigned>(3 * ((T + kWideBQ - 1) / kWideBQ)));
   rc = launch_kernel(attn_bwd_kernel<false>, grid2, dim3(kAttnThreads), st, p);
   if (rc != kOk) return rc;
   const int64_t n4 = static_cast<int64_t>(B) * NKV * per_head / 4;
@@ -1233,9 +1278,8 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_varlen_bwd
                          dim3(kAttnThreads), st, out, dout, p.delta, static_cast<int>(M), NH);
   if (rc != kOk) return rc;
   if (B > 0) {
-    const int slots = nbm;
     const dim3 grid(static_cast<unsigned>(NH), static_cast<unsigned>(B),
-                    static_cast<unsigned>(2 * slots));
+                    static_cast<unsigned>(3 * ((M + kWideBQ - 1) / kWideBQ)));
     rc = launch_kernel(attn_bwd_kernel<true>, grid, dim3(kAttnThreads), st, p);
     if (rc != kOk) return rc;
   }
