@@ -15,6 +15,7 @@ import torch
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libsoupk.so")
 _lock = threading.Lock()
 _lib = None
+_host = None     # the CPython extension (csrc/host_ops.cpp), bound to the library's entry points
 
 ABI_VERSION = 4
 STATUS_SCRATCH_LIMIT = 20001          # SOUPK_STATUS_SCRATCH_LIMIT
@@ -132,18 +133,47 @@ def lib():
             handle = load_library(_LIB_PATH)
             if torch.cuda.is_available():
                 handle.soupk_init_device()   # (a failure here resurfaces at the call)
+            _bind_host(handle)
             _lib = handle
     return _lib
 
 
-_entry = {}   # name -> the bound ctypes function of the package's library
+def _bind_host(handle):
+    """Load the host extension and give it the library's entry points."""
+    global _host
+    try:
+        from . import _soupk_host as ext
+    except ImportError as exc:
+        raise SoupkError(
+            f"the host extension beside {_LIB_PATH} is missing or does not load ({exc}): build it "
+            "with `python -m testt_amd.build_ext` (or __graft_entry__.build())") from exc
+    for name in SIGNATURES:
+        fn = getattr(handle, name)
+        if ext.bind(name, ctypes.cast(fn, ctypes.c_void_p).value):
+            _entry[name] = getattr(ext, name)
+        else:                     # (set-up and benchmark entry points stay with ctypes)
+            _entry[name] = fn
+    ext.set_status(SoupkError, ctypes.cast(handle.soupk_status_string, ctypes.c_void_p).value)
+    _host = ext
+
+
+def host():
+    """The operators of the host extension (csrc/host_ops.cpp).  Each returns None for arguments
+    outside its common case; the caller then runs its own checks."""
+    if _host is None:
+        lib()
+    return _host
+
+
+_entry = {}   # name -> the callable of the package's library entry point
 
 
 def call(name, *args):
     """Invoke entry point `name`; raise SoupkError on a non-zero status."""
     fn = _entry.get(name)
     if fn is None:
-        fn = _entry[name] = getattr(lib(), name)
+        lib()
+        fn = _entry[name]
     status = fn(*args)
     if status != 0:
         text = lib().soupk_status_string(status)

@@ -53,6 +53,9 @@ def varlen_supported(qkv, head_dim, n_heads, n_kv):
 
 def attention_varlen_fwd(qkv_r, cu_seqlens, n_heads, n_kv, scale):
     """(out [M, NH*D] fp16, lse [NH, M] fp32) of the token-major rotated rows qkv_r [M, W]."""
+    done = _ext.host().varlen_fwd(qkv_r, cu_seqlens, n_heads, n_kv, scale)
+    if done is not None:
+        return done
     _ext.require(qkv_r, "qkv_r", dtype=torch.float16, ndim=2)
     M = qkv_r.shape[0]
     dev = qkv_r.device
@@ -72,6 +75,10 @@ def attention_varlen_bwd(qkv_r, cu_seqlens, out, lse, dout, scale, n_heads, n_kv
     """dqkv [M, W] fp16: the gradient of qkv_r's rows, or -- with rope = (cos, sin, pos, batch,
     seq) (fp32 tables [>= seq, 128], int64 padded positions b*seq + t) -- of the q|k|v rows
     before the rotation, RoPE's backward applied inside the kernels."""
+    dqkv = _ext.host().varlen_bwd(qkv_r, cu_seqlens, out, lse, dout, scale, n_heads, n_kv,
+                                  *(rope if rope is not None else (None, None, None, 0, 0)))
+    if dqkv is not None:
+        return dqkv
     _ext.require(qkv_r, "qkv_r", dtype=torch.float16, ndim=2)
     M = qkv_r.shape[0]
     dev = qkv_r.device
@@ -163,6 +170,10 @@ def supported(q, k, v):
 
 def attention_fwd(q, k, v, key_valid=None, scale=None):
     """(out [B*T, NH*D] fp16, lse [B, NH, T] fp32)."""
+    done = _ext.host().attn_fwd(q, k, v, key_valid,
+                                1.0 / math.sqrt(q.shape[-1]) if scale is None else scale)
+    if done is not None:
+        return done
     B, NH, T, D = q.shape
     NKV = k.shape[1]
     dev = q.device
@@ -184,6 +195,9 @@ def attention_fwd(q, k, v, key_valid=None, scale=None):
 
 def attention_bwd(q, k, v, key_valid, out, lse, dout, scale):
     """(dq [B, NH, T, D], dk, dv [B, NKV, T, D]) fp16, from the forward's out and lse."""
+    done = _ext.host().attn_bwd(q, k, v, key_valid, out, lse, dout, scale)
+    if done is not None:
+        return done
     B, NH, T, D = q.shape
     NKV = k.shape[1]
     dev = q.device

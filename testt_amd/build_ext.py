@@ -18,6 +18,9 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB_NAME = "libsoupk.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
+HOST_SRC = os.path.join(CSRC, "host_ops.cpp")
+HOST_NAME = "_soupk_host.so"       # the CPython extension of the operators' host side
+HOST_PATH = os.path.join(HERE, HOST_NAME)
 ARCH = "gfx950"
 
 # -ffp-contract=off: products and sums are rounded one at a time (the NF4 closed form is
@@ -56,8 +59,38 @@ def _compile(hipcc, src, build_dir, defines):
     return obj
 
 
+def _build_host(hipcc, build_dir):
+    """The CPython extension, against the installed torch's headers and libraries (host code
+    only; the kernels' library is bound to it at run time, not linked)."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    obj = os.path.join(build_dir, "host_ops.o")
+    # NDEBUG: without it the headers bring a thread-local debug counter, and a library with
+    # thread-local storage loaded last sends every such access of the libraries before it (HIP
+    # makes several per launch) through the slow path of glibc before 2.39: the 64-token layer took
+    # 222 us of host time instead of 204.
+    flags = ["-x", "c++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-Wall",
+             "-D__HIP_PLATFORM_AMD__=1",
+             "-DUSE_ROCM=1",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+             f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include",
+             f"-I{sysconfig.get_paths()['include']}", "-I/opt/rocm/include"]
+    tmp = HOST_PATH + ".tmp"
+    for cmd in ([hipcc, *flags, "-c", HOST_SRC, "-o", obj],
+                [hipcc, "-shared", obj, "-o", tmp, f"-L{root}/lib", "-ltorch_python", "-ltorch",
+                 "-ltorch_cpu", "-lc10", "-lc10_hip"]):
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"building {HOST_NAME} failed:\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose=False, defines=(), out=None):
-    """Compile every kernel source and link libsoupk.so; returns the library path.
+    """Compile every kernel source and link libsoupk.so, and the host extension beside it; returns
+    the library path.
 
     `defines` (e.g. "SOUPK_HEAD_PREFETCH=8") override the launch-shape constants of the
     sources; with `out`, the library is written there instead (a tuning variant), from its
@@ -68,8 +101,11 @@ def build(verbose=False, defines=(), out=None):
     os.makedirs(build_dir, exist_ok=True)
     srcs = sources()
     jobs = max(1, min(len(srcs), os.cpu_count() or 1, 8))
-    with ThreadPoolExecutor(jobs) as pool:
+    with ThreadPoolExecutor(jobs + 1) as pool:
+        host = pool.submit(_build_host, hipcc, build_dir) if out is None else None
         objs = list(pool.map(lambda s: _compile(hipcc, s, build_dir, defines), srcs))
+        if host is not None:
+            host.result()
     tmp = lib_path + ".tmp"
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp,
            "-lhipblaslt"]

@@ -587,9 +587,9 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_fwd_wide_kernel(AttnPara
 // dK = scale * dS^T Q,  dV = P^T dO.  Three launches:
 //   attn_bwd_delta_kernel (b, head, 64 queries): D;
 //   attn_bwd_kernel       two kinds of workgroup in one grid, so that they run side by side
-//                         (of three z, two dK/dV of 64 keys and one dQ of 128 queries, the heaviest
+//                         (dK/dV of 64 keys and dQ of 64 or 128 queries in turn, the heaviest
 //                         causal blocks of both kinds dispatched first):
-//     dQ   (b, head, 128 queries): over its key blocks S^T = K Q^T, dP^T = V dO^T (the
+//     dQ   (b, head, 64 or 128 queries): over its key blocks S^T = K Q^T, dP^T = V dO^T (the
 //          forward's orientation: query = lane column), dQ^T += K^T dS^T;
 //     dKdV (b, head, 64 keys): over the query blocks that see them, S = Q K^T, dP = dO V^T
 //          (key = lane column), dV^T += dO^T P, dK^T += Q^T dS, into fp32 partials per query
@@ -720,27 +720,31 @@ __device__ __forceinline__ void store_dq(const AttnParams& p, const SeqHead& sh,
   }
 }
 
-// dQ of 128 queries: 32 per wavefront, so that every K and V fragment read from LDS serves two
-// tiles (at 16 the LDS reads of a block take as long as its MFMAs), double-buffered tiles with one
-// barrier per block, as the 128-query forward.
-template <bool VARLEN>
+// dQ of 64 U queries, 16 U per wavefront.  U = 2 (long sequences, as the 128-query forward): every K
+// and V fragment read from LDS serves two tiles (at one the LDS reads of a block take as long as its
+// MFMAs), and the tiles are double-buffered, one barrier per block; U = 1 keeps one buffer and two
+// barriers, which measured faster on short chains (rows of 512 to 128 tokens, this launch: 24.0 us
+// against 25.3 double-buffered).  A query's arithmetic is the same for both.
+template <bool VARLEN, int U>
 __device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& sh, int h,
                                                  int b, int qb, unsigned char* smem) {
   const int T = sh.len;
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int ql = lane & 15, gr = lane >> 4;
-  const int q0 = qb * kWideBQ + 32 * w;
-  const int n_kb = min(2 * qb + 2, (T + kBK - 1) / kBK);
+  const int q0 = qb * (64 * U) + 16 * U * w;
+  const int n_kb = min(U * (qb + 1), (T + kBK - 1) / kBK);
   const int kb_diag = q0 / kBK;
   const bool has_valid = sh.valid != nullptr;
   const float scale_log2 = p.scale_log2;
   constexpr int kTile = kBK * kRStride;               // halves
+  constexpr int kBufs = U == 2 ? 2 : 1;
   _Float16* const tiles = reinterpret_cast<_Float16*>(smem);    // K, V of buffer 0, then of 1
-  uint8_t* const flags = smem + 4 * kTile * 2;
-  h8 qf[2][4], dof[2][4];
-  float dsum[2], lse2[2];
+  uint8_t* const flags = smem + kBufs * 2 * kTile * 2;
+  auto buf = [](int kb) { return kBufs == 2 ? kb & 1 : 0; };
+  h8 qf[U][4], dof[U][4];
+  float dsum[U], lse2[U];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int qc = min(q0 + 16 * u + ql, T - 1);
     const uint16_t* qrow = row_at(sh.q, qc, sh.ld_q);
     const uint16_t* dorow = row_at(sh.dout, qc, sh.ld_o);
@@ -752,9 +756,9 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& 
     dsum[u] = sh.delta[qc];
     lse2[u] = sh.lse[qc] * kLog2e;   // +inf: no visible key, every p = 0
   }
-  f4 acc[2][8];
+  f4 acc[U][8];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < U; ++u)
 #pragma unroll
     for (int t = 0; t < 8; ++t) acc[u][t] = f4{0.f, 0.f, 0.f, 0.f};
   TileRegs kr, vr;
@@ -765,15 +769,15 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& 
     if (!VARLEN && has_valid) fl_raw = load_flag_raw(sh.valid, sh.k, kb * kBK, T);
   };
   auto store = [&](int kb) {
-    store_tile(tiles + (kb & 1) * 2 * kTile, kr);
-    store_tile(tiles + ((kb & 1) * 2 + 1) * kTile, vr);
+    store_tile(tiles + buf(kb) * 2 * kTile, kr);
+    store_tile(tiles + (buf(kb) * 2 + 1) * kTile, vr);
     if (!VARLEN && has_valid && threadIdx.x < kBK)
-      flags[(kb & 1) * kBK + threadIdx.x] = key_flag(fl_raw, true, kb * kBK, T);
+      flags[buf(kb) * kBK + threadIdx.x] = key_flag(fl_raw, true, kb * kBK, T);
   };
   auto block = [&](int kb, auto mask) {
-    const _Float16* K = tiles + (kb & 1) * 2 * kTile;
+    const _Float16* K = tiles + buf(kb) * 2 * kTile;
     const _Float16* V = K + kTile;
-    h8 dsb[2][2];
+    h8 dsb[U][2];
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       h8 kf[4], vf[4];
@@ -782,20 +786,20 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& 
         kf[s] = lds_h8(K + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
         vf[s] = lds_h8(V + (16 * n + ql) * kRStride + 32 * s + 8 * gr);
       }
-      f4 sc[2], dp[2];
+      f4 sc[U], dp[U];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) sc[u] = dp[u] = f4{0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < U; ++u) sc[u] = dp[u] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < U; ++u) {
           sc[u] = mfma32(kf[s], qf[u][s], sc[u]);
           dp[u] = mfma32(vf[s], dof[u][s], dp[u]);
         }
-      const uint32_t fl = !VARLEN && has_valid ? flag_word(flags + (kb & 1) * kBK, n, gr)
+      const uint32_t fl = !VARLEN && has_valid ? flag_word(flags + buf(kb) * kBK, n, gr)
                                                : 0x01010101u;
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = kb * kBK + 16 * n + 4 * gr + i;
@@ -814,37 +818,48 @@ __device__ __forceinline__ void attn_bwd_dq(const AttnParams& p, const SeqHead& 
       for (int m = 0; m < 2; ++m) {
         const h8 kt = lds_runs_tr(K, kRStride, 16 * t, m, gr);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) acc[u][t] = mfma32(kt, dsb[u][m], acc[u][t]);
+        for (int u = 0; u < U; ++u) acc[u][t] = mfma32(kt, dsb[u][m], acc[u][t]);
       }
   };
   load(0);
-  store(0);
-  __syncthreads();
+  if constexpr (kBufs == 2) {
+    store(0);
+    __syncthreads();
+  }
   for (int kb = 0; kb < n_kb; ++kb) {
+    if constexpr (kBufs == 1) {
+      __syncthreads();
+      store(kb);
+      __syncthreads();
+    }
     load(kb + 1);      // (clamped past the end)
     issue_here();
     if (kb < kb_diag && (VARLEN || !has_valid))
       block(kb, std::false_type{});
     else if (kb <= kb_diag)
       block(kb, std::true_type{});
-    store(kb + 1);
-    __syncthreads();
+    if constexpr (kBufs == 2) {
+      store(kb + 1);
+      __syncthreads();
+    }
   }
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < U; ++u) {
     const int q_abs = q0 + 16 * u + ql;
     if (q_abs < T) store_dq<VARLEN>(p, sh, h, b, q_abs, gr, acc[u]);
   }
 }
 
 // dK/dV of 64 keys, 16 per wavefront (32 would take 128 accumulator and 64 operand registers: more
-// than two wavefronts per SIMD have), double-buffered tiles and one barrier per block.  Loading the
+// than two wavefronts per SIMD have); U selects the buffers as for dQ.  Loading the
 // next 16 queries' fragments ahead of this tile's exponentials spills and doubles the time.
+template <int U>
 __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead& sh, int kb,
                                                    unsigned char* smem) {
-  constexpr int kTile = kBQ * kRStride;
+  constexpr int kTile = kBQ * kRStride, kBufs = U == 2 ? 2 : 1;
   _Float16* const tiles = reinterpret_cast<_Float16*>(smem);   // Q, dO of buffer 0, then of 1
-  float* const stats = reinterpret_cast<float*>(smem + 4 * kTile * 2);   // lse2, D of 0, of 1
+  float* const stats = reinterpret_cast<float*>(smem + kBufs * 2 * kTile * 2);   // lse2, D of 0, of 1
+  auto buf = [](int qb) { return kBufs == 2 ? qb & 1 : 0; };
   const int T = sh.len;
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int kl = lane & 15, gr = lane >> 4;
@@ -875,7 +890,7 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
     del_raw = sh.delta[t];
   };
   auto store = [&](int qb) {
-    const int bf = qb & 1;
+    const int bf = buf(qb);
     store_tile(tiles + bf * 2 * kTile, qr);
     store_tile(tiles + (bf * 2 + 1) * kTile, dr);
     if (threadIdx.x < kBQ) {
@@ -885,9 +900,9 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
     }
   };
   auto block = [&](int qb, auto mask) {
-    const _Float16* Q = tiles + (qb & 1) * 2 * kTile;
+    const _Float16* Q = tiles + buf(qb) * 2 * kTile;
     const _Float16* O = Q + kTile;
-    const float* l2s = stats + (qb & 1) * 2 * kBQ;
+    const float* l2s = stats + buf(qb) * 2 * kBQ;
     h8 pb[2], dsb[2];
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
@@ -925,17 +940,26 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
       }
   };
   load(kb);
-  store(kb);
-  __syncthreads();
+  if constexpr (kBufs == 2) {
+    store(kb);
+    __syncthreads();
+  }
   for (int qb = kb; qb < nqb; ++qb) {
+    if constexpr (kBufs == 1) {
+      __syncthreads();
+      store(qb);
+      __syncthreads();
+    }
     load(qb + 1);   // (clamped past the end)
     issue_here();
     if (qb == kb || has_valid || (qb + 1) * kBQ > T)
       block(qb, std::true_type{});
     else
       block(qb, std::false_type{});
-    store(qb + 1);
-    __syncthreads();
+    if constexpr (kBufs == 2) {
+      store(qb + 1);
+      __syncthreads();
+    }
   }
   if (key_abs >= T) return;
   float* dkp = p.dk_part + (sh.plane + key_abs) * kD;
@@ -948,26 +972,30 @@ __device__ __forceinline__ void attn_bwd_dkdv(const AttnParams& p, const SeqHead
   }
 }
 
-constexpr int kBwdLdsBytes = 4 * kBK * kRStride * 2 + 4 * kBQ * 4;
+// LDS of a workgroup: the Q and dO tiles and the lse / D values of the dK/dV kind (the larger), once
+// or twice.
+template <int U>
+constexpr int kBwdLdsBytes = U * (2 * kBK * kRStride * 2 + 2 * kBQ * 4);
 
-// Grid z = 3 * (128-query slots): z % 3 == 2 -> dQ of a 128-query block, the others dK/dV of 64 keys,
-// the heaviest causal blocks of both kinds first.  Against 64-query dQ workgroups and single LDS
-// tiles with two barriers a block (delta and reduce launches included, 12 heads, us): 2 x 4096 tokens
-// 537 -> 452, 1 x 8000 907 -> 814, rows of 4096 to 1024 477 -> 406, 4 x 1024 100 -> 94, 16 x 256 82 ->
-// 72, 4 x 512 42.2 -> 41.4, rows of 512 to 96 32.3 -> 32.5.  Bound by the dK/dV chain: 64 MFMAs, as
-// many clocks of LDS reads and 16 exponentials a block, at two wavefronts per SIMD.
-template <bool VARLEN>
+// Grid z = (U + 1) * (64 U-query slots): of U + 1 z, one dQ of 64 U queries and U dK/dV of 64 keys, the
+// heaviest causal blocks of both kinds first.  U = 2 by the 128-query forward's rule (wide_forward).
+// Against 64-query dQ workgroups on single LDS tiles with two barriers a block (delta and reduce
+// launches included, 12 heads, us): 2 x 4096 tokens 537 -> 452, 1 x 8000 907 -> 814, rows of 4096 to
+// 1024 477 -> 406, 4 x 1024 100 -> 94, 16 x 256 82 -> 72; rows of 512 to 128 tokens keep
+// U = 1 (24.0 us for this launch alone; 26.3 with U = 2).  Bound by the dK/dV chain: 64 MFMAs,
+// as many clocks of LDS reads and 16 exponentials a block, at two wavefronts per SIMD.
+template <bool VARLEN, int U>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_bwd_kernel(AttnParams p) {
-  __shared__ __align__(16) unsigned char smem[kBwdLdsBytes];
+  __shared__ __align__(16) unsigned char smem[kBwdLdsBytes<U>];
   const int h = blockIdx.x, b = blockIdx.y;
   const SeqHead sh = seq_head<VARLEN>(p, b, h);
-  const int z = static_cast<int>(blockIdx.z), zq = z / 3, zr = z - 3 * zq;
-  if (zr < 2) {
-    const int kb = 2 * zq + zr;
-    if (kb < (sh.len + kBK - 1) / kBK) attn_bwd_dkdv(p, sh, kb, smem);
+  const int z = static_cast<int>(blockIdx.z), zq = z / (U + 1), zr = z - (U + 1) * zq;
+  if (zr < U) {
+    const int kb = U * zq + zr;
+    if (kb < (sh.len + kBK - 1) / kBK) attn_bwd_dkdv<U>(p, sh, kb, smem);
   } else {
-    const int qb = (sh.len + kWideBQ - 1) / kWideBQ - 1 - zq;
-    if (qb >= 0) attn_bwd_dq<VARLEN>(p, sh, h, b, qb, smem);
+    const int qb = (sh.len + 64 * U - 1) / (64 * U) - 1 - zq;
+    if (qb >= 0) attn_bwd_dq<VARLEN, U>(p, sh, h, b, qb, smem);
   }
 }
 
@@ -1106,6 +1134,15 @@ bool wide_forward(int64_t units, int64_t len) {
   return units * ((len + kWideBQ - 1) / kWideBQ) * 4 >= int64_t{5} * device_cu_count();
 }
 
+// The dQ and dK/dV launch over block slots for sequences of up to `len` rows.
+template <bool VARLEN>
+int launch_bwd(const AttnParams& p, int32_t B, int32_t NH, int64_t len, bool wide, hipStream_t st) {
+  const int64_t z = wide ? 3 * ((len + kWideBQ - 1) / kWideBQ) : 2 * ((len + kBQ - 1) / kBQ);
+  const dim3 grid(static_cast<unsigned>(NH), static_cast<unsigned>(B), static_cast<unsigned>(z));
+  return wide ? launch_kernel(attn_bwd_kernel<VARLEN, 2>, grid, dim3(kAttnThreads), st, p)
+              : launch_kernel(attn_bwd_kernel<VARLEN, 1>, grid, dim3(kAttnThreads), st, p);
+}
+
 bool misaligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; }
 
 AttnParams base_params(int32_t NH, int32_t NKV, float scale) {
@@ -1192,9 +1229,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_bwd(
   int rc = launch_kernel(attn_bwd_delta_kernel, grid, dim3(kAttnThreads), st, out, dout,
                          p.delta, T, NH);
   if (rc != kOk) return rc;
-  const dim3 grid2(static_cast<unsigned>(NH), static_cast<unsigned>(B),
-                   static_cast<unsigned>(3 * ((T + kWideBQ - 1) / kWideBQ)));
-  rc = launch_kernel(attn_bwd_kernel<false>, grid2, dim3(kAttnThreads), st, p);
+  rc = launch_bwd<false>(p, B, NH, T, wide_forward(static_cast<int64_t>(B) * NH, T), st);
   if (rc != kOk) return rc;
   const int64_t n4 = static_cast<int64_t>(B) * NKV * per_head / 4;
   return launch_kernel(attn_bwd_reduce_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)),
@@ -1278,9 +1313,8 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_varlen_bwd
                          dim3(kAttnThreads), st, out, dout, p.delta, static_cast<int>(M), NH);
   if (rc != kOk) return rc;
   if (B > 0) {
-    const dim3 grid(static_cast<unsigned>(NH), static_cast<unsigned>(B),
-                    static_cast<unsigned>(3 * ((M + kWideBQ - 1) / kWideBQ)));
-    rc = launch_kernel(attn_bwd_kernel<true>, grid, dim3(kAttnThreads), st, p);
+    // (slots for a sequence of all M tokens)
+    rc = launch_bwd<true>(p, B, NH, M, wide_forward(static_cast<int64_t>(B) * NH, M / B), st);
     if (rc != kOk) return rc;
   }
   const int64_t items = M * NKV * 16;

@@ -209,7 +209,7 @@ def _forward_device(ctx, hidden, weight, targets, den):
     for c, start in enumerate(range(0, rows, chunk)):
         stop = min(rows, start + chunk)
         n = stop - start
-        logits = torch.matmul(hidden[start:stop], weight.t())
+        logits = _blas.linear(hidden[start:stop], weight)
         g = torch.empty((n, vocab), dtype=torch.float16, device=dev) if want_grad else None
         _ext.call("soupk_head_stats_grad_planned", logits.data_ptr(),
                   targets.data_ptr() + 8 * start,

@@ -104,13 +104,10 @@ def _f32(t):
 
 def _plan_key(weight, device):
     """What a cached plan of `weight` depends on: the addresses of its packed data and state
-    tensors and the offset object (None for an object that is not an NF4 weight)."""
-    state = _quant_state(weight)
-    try:
-        return (device, weight.data.data_ptr(), state.absmax.data_ptr(), state.code.data_ptr(),
-                state.state2.code.data_ptr(), state.state2.absmax.data_ptr(), id(state.offset))
-    except AttributeError:
-        return None
+    tensors, the offset object, the shape and the block size (None for an object that is not an
+    NF4 weight)."""
+    key = _ext.host().nf4_key(weight)
+    return None if key is None else (device, key)
 
 
 def _plan(weight, device):
@@ -214,7 +211,11 @@ def unpack_many(weights, outs):
 
 
 def unpack_concat(weights, device):
-    """fp16 [sum N_i, K]: the weights stacked by rows, unpacked in place (one launch)."""
+    """fp16 [sum N_i, K]: the weights stacked by rows, unpacked in place (one launch, its arguments
+    prepared once per list of weights: _GroupPlan)."""
+    device = torch.device(device)
+    if device.type == "cuda":
+        return unpack_groups((tuple(weights),), device)[0]
     rows = [weight_shape(w)[0] for w in weights]
     cols = weight_shape(weights[0])[1]
     out = torch.empty((sum(rows), cols), dtype=torch.float16, device=device)

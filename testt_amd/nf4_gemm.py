@@ -23,24 +23,64 @@ from . import nf4 as _nf4
 MAX_PARTS = 4
 
 
-def supported(x, weights, bias=None):
-    if not (x.is_cuda and x.dtype == torch.float16 and x.dim() == 2):
-        return False
+class _Stack:
+    """The launch arguments of one row stack of NF4 weights that the fused kernels read (1-4 parts
+    of one column count, each a multiple of 128 rows, blocksize 64, nested 256): the pointer tables
+    as ctypes arrays and their addresses in entry-point order."""
+
+    def __init__(self, weights, device):
+        plans, rows, arrays, part_rows = _nf4_args(weights, device)
+        self.rows, self.cols = sum(rows), _nf4.weight_shape(weights[0])[1]
+        self.keep = (plans, arrays, part_rows)
+        self.args = (len(weights), *[ctypes.addressof(a) for a in arrays],
+                     ctypes.addressof(part_rows), plans[0][2], plans[0][3])
+
+
+def _readable(weights, device):
+    cols = None
     if not 1 <= len(weights) <= MAX_PARTS:
         return False
-    K = x.shape[1]
     for w in weights:
         if not _nf4.supports_fast_unpack(w):
             return False
         st = w.quant_state
-        rows, cols = _nf4.weight_shape(w)
-        if cols != K or rows % 128 or st.blocksize != 64 or st.state2.blocksize != 256:
+        r, c = _nf4.weight_shape(w)
+        if r % 128 or st.blocksize != 64 or st.state2.blocksize != 256 or \
+                (cols is not None and c != cols) or _nf4._plan(w, device) is None:
             return False
-        if _nf4._plan(w, x.device) is None:
-            return False
-    if bias is not None and (bias.dtype != torch.float16 or not bias.is_cuda):
+        cols = c
+    return True
+
+
+def _stack(weights, device):
+    """The _Stack of `weights` on `device`, None where the fused kernels do not read them.  Kept on
+    the first weight and used while every weight's plan key (_nf4._plan_key) is unchanged."""
+    keys = [_nf4._plan_key(w, device) for w in weights]
+    if not keys or None in keys:
+        return None
+    cached = getattr(weights[0], "_soupk_stack", None)
+    if cached is not None and cached[0] == keys:
+        return cached[1]
+    stack = _Stack(weights, device) if _readable(weights, device) else None
+    try:
+        weights[0]._soupk_stack = (keys, stack)
+    except AttributeError:          # objects without a __dict__ are checked on every call
+        pass
+    return stack
+
+
+def _rows_fit(x, cols):
+    return (x.is_cuda and x.dtype == torch.float16 and x.dim() == 2 and x.shape[1] == cols and
+            x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0)
+
+
+def supported(x, weights, bias=None):
+    if not x.is_cuda:
         return False
-    return K % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+    st = _stack(weights, x.device)
+    if st is None or st.cols % 64 or not _rows_fit(x, st.cols):
+        return False
+    return bias is None or (bias.dtype == torch.float16 and bias.is_cuda)
 
 
 # Where the fused kernels measured ahead of unpack + hipBLASLt on MI355X (bench.py --nf4-gemm,
@@ -102,7 +142,8 @@ _cu_count.cache = {}
 def prefer_fused(x, weights):
     """True where the fused NF4 forward y = x W^T is the faster path (fused_fits)."""
     M, K = x.shape
-    N = sum(_nf4.weight_shape(w)[0] for w in weights)
+    st = _stack(weights, x.device)
+    N = st.rows if st is not None else sum(_nf4.weight_shape(w)[0] for w in weights)
     cus = _cu_count(x.device)
     return fused_fits(M, N, K, FWD_TILE, cus, forward_split_tiles(K, cus))
 
@@ -168,25 +209,10 @@ def grad_input_supported(dy, weights):
     """nf4_grad_input takes these: fp16 dy [M, N] with unit column stride and 16-byte aligned
     rows, 1-4 NF4 parts (blocksize 64, nested 256) of one column count, each a multiple of 128
     rows, W's columns a multiple of 128."""
-    if not (dy.is_cuda and dy.dtype == torch.float16 and dy.dim() == 2):
+    if not dy.is_cuda:
         return False
-    if not 1 <= len(weights) <= MAX_PARTS:
-        return False
-    cols = None
-    total = 0
-    for w in weights:
-        if not _nf4.supports_fast_unpack(w):
-            return False
-        st = w.quant_state
-        r, c = _nf4.weight_shape(w)
-        if r % 128 or st.blocksize != 64 or st.state2.blocksize != 256 or \
-                (cols is not None and c != cols):
-            return False
-        if _nf4._plan(w, dy.device) is None:
-            return False
-        cols, total = c, total + r
-    return (cols % 128 == 0 and dy.shape[1] == total and dy.stride(1) == 1 and
-            dy.stride(0) % 8 == 0 and dy.data_ptr() % 16 == 0)
+    st = _stack(weights, dy.device)
+    return st is not None and st.cols % 128 == 0 and _rows_fit(dy, st.rows)
 
 
 def nf4_grad_input(dy, weights, splits=None):
@@ -195,15 +221,14 @@ def nf4_grad_input(dy, weights, splits=None):
     `splits` cuts the contraction over W's rows (soupk_gemm_nn_nf4_split; default: split_count
     for this device and the 128 x 64 tiles)."""
     M, N = dy.shape
-    plans, rows, arrays, part_rows = _nf4_args(weights, dy.device)
-    if sum(rows) != N:
-        raise ValueError(f"dy has {N} columns, the weights {sum(rows)} rows")
-    K = _nf4.weight_shape(weights[0])[1]
+    st = _stack(weights, dy.device) or _Stack(weights, dy.device)
+    if st.rows != N:
+        raise ValueError(f"dy has {N} columns, the weights {st.rows} rows")
+    K = st.cols
     dx = torch.empty((M, K), dtype=torch.float16, device=dy.device)
     if splits is None:
         splits = split_count(M, K, N, _cu_count(dy.device), GRAD_TILE) if M > 0 else 1
-    args = (dy.data_ptr(), dy.stride(0), len(weights), *[ctypes.addressof(a) for a in arrays],
-            ctypes.addressof(part_rows), plans[0][2], plans[0][3], dx.data_ptr(), M, K, N)
+    args = (dy.data_ptr(), dy.stride(0), *st.args, dx.data_ptr(), M, K, N)
     if splits > 1:
         ws = torch.empty(_split_used(N // 64, splits)[1] * M * K, dtype=torch.float32,
                          device=dy.device)
@@ -275,29 +300,21 @@ def nf4_linear(x, weights, bias=None, splits=None):
     """x @ W^T (+ bias) for W the row stack of `weights`, dequantised in the GEMM; `splits`
     cuts the contraction (default: split_count for this device)."""
     M, K = x.shape
-    plans = [_nf4._plan(w, x.device) for w in weights]
-    rows = [_nf4.weight_shape(w)[0] for w in weights]
-    N = sum(rows)
+    st = _stack(weights, x.device) or _Stack(weights, x.device)
+    N = st.rows
     if bias is not None:
         _ext.require(bias, "bias", dtype=torch.float16, ndim=1, device=x.device)
         if bias.numel() != N:
             raise ValueError(f"bias has {bias.numel()} entries, the weights {N} rows")
-    n = len(weights)
-    arrays = [(ctypes.c_void_p * n)(*[p[0][i] for p in plans]) for i in range(6)]
-    part_rows = (ctypes.c_int32 * n)(*rows)
     y = torch.empty((M, N), dtype=torch.float16, device=x.device)
     if splits is None:
         splits = split_count(M, N, K, _cu_count(x.device)) if M > 0 else 1
     if splits > 1:
         ws = torch.empty(_split_used(K // 64, splits)[1] * M * N, dtype=torch.float32,
                          device=x.device)
-        _ext.call("soupk_gemm_tn_nf4_split", x.data_ptr(), x.stride(0), n,
-                  *[ctypes.addressof(a) for a in arrays], ctypes.addressof(part_rows),
-                  plans[0][2], plans[0][3], _ext.ptr(bias), y.data_ptr(), M, N, K, splits,
-                  ws.data_ptr(), ws.numel(), _ext.stream_of(x))
+        _ext.call("soupk_gemm_tn_nf4_split", x.data_ptr(), x.stride(0), *st.args, _ext.ptr(bias),
+                  y.data_ptr(), M, N, K, splits, ws.data_ptr(), ws.numel(), _ext.stream_of(x))
         return y
-    _ext.call("soupk_gemm_tn_nf4", x.data_ptr(), x.stride(0), n,
-              *[ctypes.addressof(a) for a in arrays], ctypes.addressof(part_rows),
-              plans[0][2], plans[0][3], _ext.ptr(bias), y.data_ptr(), M, N, K,
-              _ext.stream_of(x))
+    _ext.call("soupk_gemm_tn_nf4", x.data_ptr(), x.stride(0), *st.args, _ext.ptr(bias),
+              y.data_ptr(), M, N, K, _ext.stream_of(x))
     return y

@@ -28,6 +28,13 @@ def _weight32(weight, hidden, device):
 
 def _launch_fwd(x, delta, weight, eps, pad_idx, padded_rows):
     """(s, y16, ypad32, rstd) of solution/rmsnorm.py:76-92."""
+    inv = None
+    if pad_idx is not None and pad_idx.dtype is torch.int64 and pad_idx.dim() == 1 and \
+            pad_idx.is_cuda and pad_idx.numel() != padded_rows:
+        inv = inverse_map(pad_idx.contiguous(), int(padded_rows))
+    done = _ext.host().rmsnorm_fwd(x, delta, weight, eps, pad_idx, int(padded_rows or 0), inv)
+    if done is not None:
+        return done
     _ext.require(x, "x", dtype=torch.float32, ndim=2)
     rows, hidden = x.shape
     dev = x.device
@@ -64,6 +71,10 @@ def _launch_fwd(x, delta, weight, eps, pad_idx, padded_rows):
 
 def _launch_bwd(s, rstd, weight, pad_idx, grad_s, grad_y, grad_ypad, want_delta):
     """(dx, ddelta or None) of solution/rmsnorm.py:95-112."""
+    done = _ext.host().rmsnorm_bwd(s, rstd, weight, pad_idx, grad_s, grad_y, grad_ypad,
+                                   bool(want_delta))
+    if done is not None:
+        return done
     _ext.require(s, "s", dtype=torch.float32, ndim=2)
     rows, hidden = s.shape
     dev = s.device

@@ -48,6 +48,15 @@ def _lora_pair(lora_q, lora_v):
 class RopePack(torch.autograd.Function):
     @staticmethod
     def forward(ctx, qkv, lora_q, lora_v, cos, sin, pos_idx, batch, seq, n_heads, n_kv, head_dim):
+        if pos_idx.dtype is torch.int64 and pos_idx.is_cuda and pos_idx.dim() == 1:
+            rows, slots = pos_idx.numel(), batch * seq
+            inv = inverse_map(pos_idx.contiguous(), slots) if rows != slots else None
+            done = _ext.host().rope_fwd(qkv, lora_q, lora_v, cos, sin, pos_idx, inv, batch, seq,
+                                        n_heads, n_kv, head_dim)
+            if done is not None:
+                ctx.save_for_backward(cos, sin, pos_idx)
+                ctx.dims = (rows, batch, seq, n_heads, n_kv, head_dim)
+                return done
         _ext.require(qkv, "qkv", dtype=torch.float16, ndim=2)
         rows = qkv.shape[0]
         dev = qkv.device
@@ -90,10 +99,14 @@ class RopePack(torch.autograd.Function):
         if not (need_qkv or need_lq or need_lv):
             return (None,) * 11
         width = (n_heads + 2 * n_kv) * head_dim
-        dqkv = torch.empty((rows, width), dtype=torch.float16, device=pos_idx.device)
-        grads = [g.to(torch.float16).contiguous() if g is not None else None
-                 for g in (grad_q, grad_k, grad_v)]
-        if rows:
+        dqkv = _ext.host().rope_bwd(grad_q, grad_k, grad_v, cos, sin, pos_idx, batch, seq,
+                                    n_heads, n_kv, head_dim)
+        launched = dqkv is not None
+        if not launched:
+            dqkv = torch.empty((rows, width), dtype=torch.float16, device=pos_idx.device)
+            grads = [g.to(torch.float16).contiguous() if g is not None else None
+                     for g in (grad_q, grad_k, grad_v)]
+        if rows and not launched:
             _ext.call("soupk_rope_pack_bwd", _ext.ptr(grads[0]), _ext.ptr(grads[1]),
                       _ext.ptr(grads[2]), _ext.ptr(cos), _ext.ptr(sin), _ext.ptr(pos_idx),
                       _ext.ptr(dqkv), rows, batch, seq, n_heads, n_kv, head_dim,
@@ -122,6 +135,11 @@ def rope_pack_tokens(qkv, lora_q, lora_v, cos, sin, pos_idx, batch, seq, n_heads
     real tokens where they are (no padded layout, no zero rows).  head_dim 128.  A token whose
     position lies outside [0, batch*seq) gets a row of zeros.  Not differentiable by itself:
     attention.RopeAttention carries its backward (fused into the attention backward)."""
+    if head_dim == 128:
+        out = _ext.host().rope_tokens(qkv, lora_q, lora_v, cos, sin, pos_idx, batch, seq, n_heads,
+                                      n_kv)
+        if out is not None:
+            return out, cos, sin, pos_idx
     _ext.require(qkv, "qkv", dtype=torch.float16, ndim=2)
     rows = qkv.shape[0]
     dev = qkv.device
