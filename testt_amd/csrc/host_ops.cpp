@@ -4,8 +4,9 @@
 //
 // Reason: a training program's small calls are bound by the host.  Through ctypes an entry point of
 // 16 arguments costs about 2 us more than its launch, and the checks and torch.empty calls around it
-// 10 - 20 us of Python.  Eager forward + backward on the MI355X box (us, before / after):
-// @table@
+// 10 - 20 us of Python.  Eager forward + backward on MI355X, before and after (us): add + RMSNorm of 300
+// rows 49 / 36, q|k|v projection of 16 rows 71 / 51, RoPE + attention of rows of 512 to 128 tokens 67
+// / 49, the padded form 122 / 95.
 //
 // An operator here takes only the common case -- plain tensors of the expected types, contiguous, on
 // one device, with matching shapes -- and returns None for anything else; the Python caller then
