@@ -581,6 +581,15 @@ constexpr int kBM = Shape::BM, kBN = Shape::BN;
 using SmallShape = GemmShape<32, 128, 1, 4>;
 constexpr int kSmallRows = 32;
 static_assert(SmallShape::BN == kBN && SmallShape::BK == kBK, "one column tiling for both");
+// From 33 to 64 rows half of the 128-row tile was copies of the last row; 64-row tiles on 8
+// wavefronts of 32 x 32 read each decoded W fragment for half the matrix work.  Measured (MI355X,
+// NF4 W, eight stacks in turn): gate|up 33 rows 23.6 -> 20.1 us, 64 rows 23.1 -> 18.8, down
+// 64 rows 16.0 -> 14.4, q|k|v and o about 1 us less.  The line lies at the tile: past 64 rows
+// they would take two row tiles, which decode W twice.  Same products in the same order:
+// identical results.
+using MidShape = GemmShape<64, 128, 2, 4>;
+constexpr int kMidRows = MidShape::BM;
+static_assert(MidShape::BN == kBN && MidShape::BK == kBK, "one column tiling for all");
 
 int check_gemm(int64_t M, int32_t N, int32_t K, int64_t ldx) {
   if (M < 0 || N <= 0 || K <= 0 || N % kBN || K % kBK || ldx < K || ldx % 8) return kInvalid;
@@ -701,6 +710,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_tn_nf4(
                          dim3(static_cast<unsigned>(N / kBN)), dim3(SmallShape::kThreads),
                          static_cast<hipStream_t>(stream), x, ldx, nullptr, nw, bias, y,
                          static_cast<int>(M), N, K, nullptr, K / kBK);
+  if (M <= kMidRows)
+    return launch_kernel(gemm_tn_kernel<MidShape, true>,
+                         dim3(static_cast<unsigned>(N / kBN)), dim3(MidShape::kThreads),
+                         static_cast<hipStream_t>(stream), x, ldx, nullptr, nw, bias, y,
+                         static_cast<int>(M), N, K, nullptr, K / kBK);
   const dim3 grid(static_cast<unsigned>((N / kBN) * ((M + kBM - 1) / kBM)));
   return launch_kernel(gemm_tn_kernel<Shape, true>, grid, dim3(Shape::kThreads),
                        static_cast<hipStream_t>(stream), x, ldx, nullptr, nw, bias, y,
@@ -733,6 +747,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_tn_nf4_split(
     r = launch_kernel(gemm_tn_kernel<SmallShape, true>,
                       dim3(static_cast<unsigned>(N / kBN), static_cast<unsigned>(used)),
                       dim3(SmallShape::kThreads), st, x, ldx, nullptr, nw, bias, y,
+                      static_cast<int>(M), N, K, workspace, per);
+  else if (M <= kMidRows)
+    r = launch_kernel(gemm_tn_kernel<MidShape, true>,
+                      dim3(static_cast<unsigned>(N / kBN), static_cast<unsigned>(used)),
+                      dim3(MidShape::kThreads), st, x, ldx, nullptr, nw, bias, y,
                       static_cast<int>(M), N, K, workspace, per);
   else
     r = launch_kernel(gemm_tn_kernel<Shape, true>,
@@ -775,6 +794,11 @@ using NS = GemmShape<128, 64, 4, 2>;
 using NSmall = GemmShape<32, 64, 1, 2>;
 static_assert(NSmall::BN == NS::BN, "one column tiling for both");
 constexpr int kNnSmallRows = SOUPK_GEMM_NN_SMALL ? 32 : 0;
+// Up to 64 rows (the split form: 33 to 64), 64-row tiles on 4 wavefronts of 32 x 32, as in the
+// forward.  Measured (MI355X): at 64 rows gate|up 24.5 -> 20.9 us, down (unsplit) 19.5 -> 18.5,
+// q|k|v and o about 1 us less.  Identical results.
+using NMid = GemmShape<64, 64, 2, 2>;
+static_assert(NMid::BN == NS::BN && NMid::BM == kMidRows, "one column tiling, one line");
 
 // The input gradient's arguments, checked; N: W's columns (dx's), K: W's rows (the
 // contraction, dy's columns).
@@ -803,6 +827,10 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4(
   if (rc != kOk) return rc;
   if (M == 0) return kOk;
   if (bad_ptr(dy) || bad_ptr(dx)) return kInvalid;
+  if (M <= kMidRows)
+    return launch_kernel(gemm_nn_nf4_kernel<NMid>, dim3(static_cast<unsigned>(N / NS::BN)),
+                         dim3(NMid::kThreads), static_cast<hipStream_t>(stream), dy, lddy, nw, dx,
+                         static_cast<int>(M), N, K, nullptr, K / 64);
   const dim3 grid(static_cast<unsigned>((N / NS::BN) * ((M + NS::BM - 1) / NS::BM)));
   return launch_kernel(gemm_nn_nf4_kernel<NS>, grid, dim3(NS::kThreads),
                        static_cast<hipStream_t>(stream), dy, lddy, nw, dx, static_cast<int>(M),
@@ -830,6 +858,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4_split(
     r = launch_kernel(gemm_nn_nf4_kernel<NSmall>,
                       dim3(static_cast<unsigned>(N / NS::BN), static_cast<unsigned>(used)),
                       dim3(NSmall::kThreads), st, dy, lddy, nw, dx, static_cast<int>(M), N, K,
+                      workspace, per);
+  else if (M <= kMidRows)
+    r = launch_kernel(gemm_nn_nf4_kernel<NMid>,
+                      dim3(static_cast<unsigned>(N / NS::BN), static_cast<unsigned>(used)),
+                      dim3(NMid::kThreads), st, dy, lddy, nw, dx, static_cast<int>(M), N, K,
                       workspace, per);
   else
     r = launch_kernel(gemm_nn_nf4_kernel<NS>,
