@@ -235,3 +235,19 @@ def test_fused_lora_rope_layer_matches_unfused(monkeypatch, lengths):
                                                                               *w.lora_v)])
     for name, a, b in zip(("s", "d", "ds", "dd", "dA_q", "dB_q", "dA_v", "dB_v"), *results):
         assert torch.equal(a.detach(), b.detach()), name
+
+
+@pytest.mark.parametrize("M", [16, 257, 600, 2100, 4100])
+def test_lora_row_counts(M):
+    """Row counts at which the column split differs (7, 7, 6, 1 and 1 parts of the output): the
+    RoPE form against lora_fwd and the RoPE pack bit for bit, and the row backward against
+    float64, as the tests above state them."""
+    test_lora_rope_fwd_matches_lora_then_rope((M - 5, 5), M, 12, 2, 2.0)
+    test_lora_bwd_rows(M, 1536, 1536, 256, 2.0, True)
+
+
+@pytest.mark.parametrize("M", [3071, 3072, 6144, 6401])
+def test_lora_bwd_params_slices(M):
+    """The last row count of 128-row slices, the first of 256- and of 512-row slices, and a last
+    slice of one row."""
+    test_lora_bwd_params(M, 512, 512, 256, 2.0, True)

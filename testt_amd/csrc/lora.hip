@@ -27,10 +27,10 @@
 //
 // A workgroup is 4 wavefronts and kRowTiles 16-row MFMA tiles (which share every A / B fragment a
 // wavefront loads), and the workgroups of a row block split the wide output (lq|lv, or dy) by
-// 16-column tiles (grid.y parts), each recomputing the block's rank-2r product (the rank-2r
-// product, t or dt, and gs are written by part 0).  Measured on MI355X at 2048 rows: one row tile
-// and about 256 workgroups (two column parts) is fastest (13.3 / 11.2 us against 16.4 / 13.8 us
-// with one part; four row tiles, or more parts, are slower).  The long contractions (over H for t,
+// tiles of columns (grid.y parts), each recomputing the block's rank-2r product (t or dt is
+// written by part 0).  Measured on MI355X at 2048 rows: one row tile and 256 workgroups (two
+// column parts) is fastest (13.3 / 11.2 us against 16.4 / 13.8 us with one part; two or four row
+// tiles, or more parts, are slower; at 16000 rows two row tiles would be level for the RoPE form).  The long contractions (over H for t,
 // over NQ / NV for dt) run on v_mfma_f32_16x16x32_f16 with the contraction split over the 4
 // wavefronts and the partial sums added in wavefront order (deterministic).  The short ones (over r
 // for lq/lv, on v_mfma_f32_16x16x16f16; over 2r for dy, on 16x16x32) are computed transposed, one
@@ -108,11 +108,16 @@ __global__ __launch_bounds__(256) void lora_stage_kernel(LoraStageArgs a) {
 // rows the varlen attention reads, out = [rotated q + lq | rotated k | v + lv] in the q|k|v
 // GEMM's own layout [M, NQ + NK + NV] (head dim 128), with the arithmetic of
 // soupk_rope_pack_tokens: x = fp32(qkv) + fp32(fp16 LoRA delta), then
-// (x1*c1 - x2*s1, x2*c2 + x1*s2) with each product rounded, then fp16.  The LoRA tiles of a
-// head's dims d..d+15 and d+64..d+79 (the rotation partners) are tiles j and j + 4 of the head's
-// eight, which the same wavefront computes as items u and u + 1 of a batch (a wavefront takes
-// every fourth tile, and the column parts split the tiles at whole heads), so a lane holds
-// both partners of its four dims.  The k columns are extra tiles with no LoRA product.
+// (x1*c1 - x2*s1, x2*c2 + x1*s2) with each product rounded, then fp16.  Two wavefronts share a
+// head, each 32 of the dims below 64 and their rotation partners (+ 64), as two MFMA tiles each.
+// Operand row ql of tile u is column 8(ql/4) + 4u + ql%4 of the 32, so a lane holds 8 consecutive
+// columns of one row and their partners: 16-byte loads and stores, 64 bytes of a row together.
+// With 16 consecutive columns per tile (8-byte accesses, 32 bytes of a row, written past the
+// caches as part lines) the kernel took 52.7 us at 8192 rows, 15.9 at 2048 and 17.0 at 888;
+// with these accesses, cached stores and the position and table loads ahead of the first
+// product 31.0, 12.8 and 15.1 (888 rows: 10.2 with the split of column_parts), identical bits.
+// Memory floor at 8192 rows: 92 MB, 14 us; what is left is one workgroup's chain of loads (two
+// are resident per CU).  The k heads have no LoRA product.
 struct LoraRope {
   const uint16_t* qkv;   // [M, W] q|k|v GEMM output, W = NQ + NK + NV
   uint16_t* out;         // [M, W]
@@ -143,41 +148,75 @@ __global__ __launch_bounds__(kThreads) void lora_fwd_kernel(
   const int nq16 = NQ / 16;
   const int nlora = NQ / 16 + NV / 16;
   int t_begin, n16;
-  if constexpr (ROPE) {   // whole heads (8 tiles) per column part
+  if constexpr (ROPE) {   // whole heads per column part; two wavefronts per head
     const int heads = (nlora + ra.NK / 16) / 8;
-    t_begin = 8 * tile_part(heads, blockIdx.y, gridDim.y);
-    n16 = 8 * tile_part(heads, blockIdx.y + 1, gridDim.y);
+    t_begin = tile_part(heads, blockIdx.y, gridDim.y) + (w >> 1);
+    n16 = tile_part(heads, blockIdx.y + 1, gridDim.y);
   } else {
-    t_begin = tile_part(nlora, blockIdx.y, gridDim.y);
+    t_begin = tile_part(nlora, blockIdx.y, gridDim.y) + w;
     n16 = tile_part(nlora, blockIdx.y + 1, gridDim.y);
   }
+  constexpr int kStep = ROPE ? 2 : 4 * kBatch;   // heads, or tiles, per round of the wavefronts
   const int W = NQ + ra.NK + NV;
-  // (ROPE) the output column of tile `tile`: q tiles, then v tiles, then k tiles
-  auto tile_col = [&](int tile) {
-    return tile < nq16 ? 16 * tile
-                       : (tile < nlora ? NQ + ra.NK + 16 * (tile - nq16) : NQ + 16 * (tile - nlora));
+  const int nq_heads = NQ / 128, nlora_heads = nlora / 8;
+  const int d0 = 32 * (w & 1) + 8 * gr;   // (ROPE) this lane's dims d0 .. d0+7, and those + 64
+  // (ROPE) the first output column of head `h`: q heads, then v heads, then k heads
+  auto head_col = [&](int h) {
+    return h < nq_heads ? 128 * h
+                        : (h < nlora_heads ? NQ + ra.NK + 128 * (h - nq_heads)
+                                           : NQ + 128 * (h - nlora_heads));
   };
-  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
-  auto load_b = [&](h4* bw, u32x2v (*xq)[kRowTiles], int t0) {
+  auto load_b = [&](h4* bw, u32x4 (*xq)[kRowTiles], int t0) {
+    if constexpr (ROPE) {
+      const int h = min(t0, n16 - 1), hb = min(h, nlora_heads - 1);
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      // B16 row of output tile column ql (the v rows follow the q rows)
-      const int tile = min(t0 + 4 * u, max(n16 - 1, 0));
-      const int bt = ROPE ? min(tile, nlora - 1) : tile;
-      bw[u] = *reinterpret_cast<const h4*>(b16 + static_cast<int64_t>(16 * bt + ql) * kR +
-                                           4 * gr);
-      if constexpr (ROPE) {   // this lane's four columns of the GEMM output
+      for (int u = 0; u < 4; ++u) {
+        const int c = 64 * (u >> 1) + 32 * (w & 1) + 8 * (ql >> 2) + 4 * (u & 1) + (ql & 3);
+        bw[u] = *reinterpret_cast<const h4*>(b16 + static_cast<int64_t>(128 * hb + c) * kR +
+                                             4 * gr);
+      }
 #pragma unroll
-        for (int rt = 0; rt < kRowTiles; ++rt) {
-          const int64_t m = min(m0 + 16 * rt + ql, M - 1);
-          xq[u][rt] = *reinterpret_cast<const u32x2v*>(ra.qkv + m * W + tile_col(tile) + 4 * gr);
-        }
+      for (int rt = 0; rt < kRowTiles; ++rt) {
+        const uint16_t* src =
+            ra.qkv + static_cast<int64_t>(min(m0 + 16 * rt + ql, M - 1)) * W + head_col(h) + d0;
+        xq[0][rt] = *reinterpret_cast<const u32x4*>(src);
+        xq[1][rt] = *reinterpret_cast<const u32x4*>(src + 64);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        // B16 row of output tile column ql (the v rows follow the q rows)
+        const int tile = min(t0 + 4 * u, max(n16 - 1, 0));
+        bw[u] = *reinterpret_cast<const h4*>(b16 + static_cast<int64_t>(16 * tile + ql) * kR +
+                                             4 * gr);
       }
     }
   };
   h4 bw_next[kBatch];
-  u32x2v xq_next[kBatch][kRowTiles];
-  if (t_begin + w < n16) load_b(bw_next, xq_next, t_begin + w);
+  u32x4 xq_next[2][kRowTiles];
+  // (ROPE) per lane: the position of its rows and the table entries of its dims (the same of
+  // every head), loaded now: the position and the tables are two loads in a row that would
+  // otherwise be waited for between t and the first output
+  f4 cs1[kRowTiles][2], cs2[kRowTiles][2], sn1[kRowTiles][2], sn2[kRowTiles][2];
+  bool pos_ok[kRowTiles];
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int rt = 0; rt < kRowTiles; ++rt) {
+      const int64_t p = ra.pos[min(m0 + 16 * rt + ql, M - 1)];
+      pos_ok[rt] = p >= 0 && p < ra.slots;
+      const uint32_t pu = pos_ok[rt] ? static_cast<uint32_t>(p) : 0u;
+      const uint32_t t = pu - ra.per_seq.div(pu) * static_cast<uint32_t>(ra.T);
+      const int64_t e = static_cast<int64_t>(t) * 128 + d0;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        cs1[rt][q] = *reinterpret_cast<const f4*>(ra.cos_t + e + 4 * q);
+        cs2[rt][q] = *reinterpret_cast<const f4*>(ra.cos_t + e + 64 + 4 * q);
+        sn1[rt][q] = *reinterpret_cast<const f4*>(ra.sin_t + e + 4 * q);
+        sn2[rt][q] = *reinterpret_cast<const f4*>(ra.sin_t + e + 64 + 4 * q);
+      }
+    }
+  }
+  if (t_begin < n16) load_b(bw_next, xq_next, t_begin);
   // t = y A^T: A operand = y rows (row 16rt + ql of row tile rt, k = k0 + 8gr..+7); B operand =
   // A_q / A_v rows (column = feature ql), loaded once per step for the kRowTiles row tiles.
   // The contraction over H is split over the 4 wavefronts; batches of kBatch steps, the next
@@ -271,24 +310,6 @@ __global__ __launch_bounds__(kThreads) void lora_fwd_kernel(
                  static_cast<_Float16>(tv[2]), static_cast<_Float16>(tv[3])};
     row_ok[rt] = m0 + 16 * rt + ql < M;
   }
-  // (ROPE) per lane: the position of its rows and the table entries of its dims d .. d+3 and
-  // d+64 .. d+67, d = 16w + 4gr (every tile pair this wavefront takes is j = w, j + 4 of a head)
-  f4 cs1[kRowTiles], cs2[kRowTiles], sn1[kRowTiles], sn2[kRowTiles];
-  bool pos_ok[kRowTiles];
-  if constexpr (ROPE) {
-#pragma unroll
-    for (int rt = 0; rt < kRowTiles; ++rt) {
-      const int64_t p = ra.pos[min(m0 + 16 * rt + ql, M - 1)];
-      pos_ok[rt] = p >= 0 && p < ra.slots;
-      const uint32_t pu = pos_ok[rt] ? static_cast<uint32_t>(p) : 0u;
-      const uint32_t t = pu - ra.per_seq.div(pu) * static_cast<uint32_t>(ra.T);
-      const int64_t e = static_cast<int64_t>(t) * 128 + 16 * w + 4 * gr;
-      cs1[rt] = *reinterpret_cast<const f4*>(ra.cos_t + e);
-      cs2[rt] = *reinterpret_cast<const f4*>(ra.cos_t + e + 64);
-      sn1[rt] = *reinterpret_cast<const f4*>(ra.sin_t + e);
-      sn2[rt] = *reinterpret_cast<const f4*>(ra.sin_t + e + 64);
-    }
-  }
   // fp16(fp16(c) * scaling), the LoRA delta as peft's fp16 matmul and scaling round it (the
   // empty asm keeps the multiply and the fp16 conversion from fusing into one rounding)
   auto delta = [&](float c) {
@@ -296,24 +317,25 @@ __global__ __launch_bounds__(kThreads) void lora_fwd_kernel(
     asm("" : "+v"(v));
     return r16(v);
   };
-  auto out_tiles = [&](const h4* bw, u32x2v (*xq)[kRowTiles], int t0) {
+  auto out_tiles = [&](const h4* bw, u32x4 (*xq)[kRowTiles], int t0) {
     if constexpr (ROPE) {
-      const StreamOut out(ra.out, static_cast<uint64_t>(M) * W * 2u);
+      // (cached stores: a wavefront's 64 bytes of a row are half a line)
+      const StreamOutT<0> out(ra.out, static_cast<uint64_t>(M) * W * 2u);
+      const bool is_q = t0 < nq_heads, is_k = t0 >= nlora_heads;
+      const int col = head_col(t0) + d0;
 #pragma unroll
-      for (int pr = 0; pr < kBatch / 2; ++pr) {
-        const int tile = t0 + 8 * pr;          // dims d of a head; tile + 4: dims d + 64
-        if (tile >= n16) break;
-        const bool is_q = tile < nq16, is_k = tile >= nlora;
-        const int col = tile_col(tile);
+      for (int rt = 0; rt < kRowTiles; ++rt) {
+        const h4 tr = is_q ? tq4[rt] : tv4[rt];
+        u32x4 o1, o2;
 #pragma unroll
-        for (int rt = 0; rt < kRowTiles; ++rt) {
-          const u32x2v a2 = xq[2 * pr][rt], b2 = xq[2 * pr + 1][rt];
-          float x1[4] = {lo_h(a2.x), hi_h(a2.x), lo_h(a2.y), hi_h(a2.y)};
-          float x2[4] = {lo_h(b2.x), hi_h(b2.x), lo_h(b2.y), hi_h(b2.y)};
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t a0 = xq[0][rt][2 * q], a1 = xq[0][rt][2 * q + 1];
+          const uint32_t b0 = xq[1][rt][2 * q], b1 = xq[1][rt][2 * q + 1];
+          float x1[4] = {lo_h(a0), hi_h(a0), lo_h(a1), hi_h(a1)};
+          float x2[4] = {lo_h(b0), hi_h(b0), lo_h(b1), hi_h(b1)};
           if (!is_k) {
-            const h4 tr = is_q ? tq4[rt] : tv4[rt];
-            const f4 c1 = mfma16(bw[2 * pr], tr, f4{0.f, 0.f, 0.f, 0.f});
-            const f4 c2 = mfma16(bw[2 * pr + 1], tr, f4{0.f, 0.f, 0.f, 0.f});
+            const f4 c1 = mfma16(bw[q], tr, f4{0.f, 0.f, 0.f, 0.f});
+            const f4 c2 = mfma16(bw[2 + q], tr, f4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               x1[i] = x1[i] + delta(c1[i]);
@@ -323,8 +345,8 @@ __global__ __launch_bounds__(kThreads) void lora_fwd_kernel(
           if (is_q || is_k) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const float r1 = x1[i] * cs1[rt][i] - x2[i] * sn1[rt][i];
-              const float r2 = x2[i] * cs2[rt][i] + x1[i] * sn2[rt][i];
+              const float r1 = x1[i] * cs1[rt][q][i] - x2[i] * sn1[rt][q][i];
+              const float r2 = x2[i] * cs2[rt][q][i] + x1[i] * sn2[rt][q][i];
               x1[i] = r1;
               x2[i] = r2;
             }
@@ -333,12 +355,15 @@ __global__ __launch_bounds__(kThreads) void lora_fwd_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) x1[i] = x2[i] = 0.f;
           }
-          if (row_ok[rt]) {
-            const uint32_t off =
-                (static_cast<uint32_t>(m0 + 16 * rt + ql) * W + col + 4 * gr) * 2u;
-            out.store(off, u32x2{pack_h2(x1[0], x1[1]), pack_h2(x1[2], x1[3])});
-            out.store(off + 128u, u32x2{pack_h2(x2[0], x2[1]), pack_h2(x2[2], x2[3])});
-          }
+          o1[2 * q] = pack_h2(x1[0], x1[1]);
+          o1[2 * q + 1] = pack_h2(x1[2], x1[3]);
+          o2[2 * q] = pack_h2(x2[0], x2[1]);
+          o2[2 * q + 1] = pack_h2(x2[2], x2[3]);
+        }
+        if (row_ok[rt]) {
+          const uint32_t off = (static_cast<uint32_t>(m0 + 16 * rt + ql) * W + col) * 2u;
+          out.store(off, o1);
+          out.store(off + 128u, o2);
         }
       }
     } else {
@@ -366,27 +391,28 @@ __global__ __launch_bounds__(kThreads) void lora_fwd_kernel(
     }
   };
   h4 bw_cur[kBatch];
-  u32x2v xq_cur[kBatch][kRowTiles];
+  u32x4 xq_cur[2][kRowTiles];
   auto take = [&]() {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      bw_cur[u] = bw_next[u];
-      if constexpr (ROPE) {
+    for (int u = 0; u < kBatch; ++u) bw_cur[u] = bw_next[u];
+    if constexpr (ROPE) {
 #pragma unroll
-        for (int rt = 0; rt < kRowTiles; ++rt) xq_cur[u][rt] = xq_next[u][rt];
+      for (int rt = 0; rt < kRowTiles; ++rt) {
+        xq_cur[0][rt] = xq_next[0][rt];
+        xq_cur[1][rt] = xq_next[1][rt];
       }
     }
   };
-  for (int t0 = t_begin + w; t0 < n16; t0 += 8 * kBatch) {
+  for (int t0 = t_begin; t0 < n16; t0 += 2 * kStep) {
     take();
-    if (t0 + 4 * kBatch < n16) load_b(bw_next, xq_next, t0 + 4 * kBatch);
+    if (t0 + kStep < n16) load_b(bw_next, xq_next, t0 + kStep);
     issue_here();
     out_tiles(bw_cur, xq_cur, t0);
-    if (t0 + 4 * kBatch < n16) {
+    if (t0 + kStep < n16) {
       take();
-      if (t0 + 8 * kBatch < n16) load_b(bw_next, xq_next, t0 + 8 * kBatch);
+      if (t0 + 2 * kStep < n16) load_b(bw_next, xq_next, t0 + 2 * kStep);
       issue_here();
-      out_tiles(bw_cur, xq_cur, t0 + 4 * kBatch);
+      out_tiles(bw_cur, xq_cur, t0 + kStep);
     }
   }
 }
@@ -486,53 +512,58 @@ __global__ __launch_bounds__(kThreads) void lora_bwd_rows_kernel(
       dt_out[static_cast<int64_t>(m0 + m) * (2 * kR) + f] = h_bits(h);
   }
   __syncthreads();
-  // dy = dt A16 (contraction over the 2r rank indices; A = A_q rows then A_v rows), one
-  // 16-column tile of H at a time, transposed: A operand = A16 columns (row h0 + ql, k = rank
-  // 8gr..+7: 8 consecutive entries of row h0 + ql of A16T, one 16-byte load), B = dt rows
-  // (column = row ql of a row tile)
+  // dy = dt A16 (contraction over the 2r rank indices; A = A_q rows then A_v rows), 32 columns
+  // of H at a time as two transposed tiles: A operand = A16 columns (k = rank 8gr..+7: 8
+  // consecutive entries of a row of A16T, one 16-byte load), B = dt rows (column = row ql of a
+  // row tile).  Operand row ql of tile u is column 8(ql/4) + 4u + ql%4 of the 32, so that a lane
+  // ends with 8 consecutive columns of one row (one 16-byte store, 64 bytes of a row together).
   h8 dtb[kRowTiles];
 #pragma unroll
   for (int rt = 0; rt < kRowTiles; ++rt) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) dtb[rt][i] = static_cast<_Float16>(dts[16 * rt + ql][8 * gr + i]);
   }
-  const _Float16* abase = staged + L.a16t + static_cast<int64_t>(ql) * (2 * kR) + 8 * gr;
-  const int t_begin = tile_part(H / 16, blockIdx.y, gridDim.y);
-  const int n16 = tile_part(H / 16, blockIdx.y + 1, gridDim.y);
+  const _Float16* abase =
+      staged + L.a16t + static_cast<int64_t>(8 * (ql >> 2) + (ql & 3)) * (2 * kR) + 8 * gr;
+  constexpr int kPairs = kBatch / 2;      // 32-column pairs per batch of a wavefront
+  const int t_begin = tile_part(H / 32, blockIdx.y, gridDim.y);
+  const int n32 = tile_part(H / 32, blockIdx.y + 1, gridDim.y);
   auto load_a = [&](h8* araw, int t0) {
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const int h0 = 16 * min(t0 + 4 * u, n16 - 1);
+      const int h0 = 32 * min(t0 + 4 * (u >> 1), n32 - 1) + 4 * (u & 1);
       araw[u] = *reinterpret_cast<const h8*>(abase + static_cast<int64_t>(h0) * (2 * kR));
     }
   };
   auto out_tiles = [&](const h8* araw, int t0) {
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
+    for (int u = 0; u < kPairs; ++u) {
       const int tile = t0 + 4 * u;
-      if (tile >= n16) break;
-      const h8 a = araw[u];
+      if (tile >= n32) break;
 #pragma unroll
       for (int rt = 0; rt < kRowTiles; ++rt) {
-        const f4 c = mfma32(a, dtb[rt], f4{0.f, 0.f, 0.f, 0.f});
+        const f4 c = mfma32(araw[2 * u], dtb[rt], f4{0.f, 0.f, 0.f, 0.f});
+        const f4 d = mfma32(araw[2 * u + 1], dtb[rt], f4{0.f, 0.f, 0.f, 0.f});
         if (row_ok[rt])
-          *reinterpret_cast<u32x2*>(dy + (m0 + 16 * rt + ql) * static_cast<int64_t>(H) +
-                                    16 * tile + 4 * gr) =
-              u32x2{pack_h2(c[0], c[1]), pack_h2(c[2], c[3])};
+          *reinterpret_cast<u32x4*>(dy + (m0 + 16 * rt + ql) * static_cast<int64_t>(H) +
+                                    32 * tile + 8 * gr) =
+              u32x4{pack_h2(c[0], c[1]), pack_h2(c[2], c[3]), pack_h2(d[0], d[1]),
+                    pack_h2(d[2], d[3])};
       }
     }
   };
-  if (t_begin + w < n16) {
+  constexpr int kStep = 4 * kPairs;
+  if (t_begin + w < n32) {
     h8 a0[kBatch], a1[kBatch];
     load_a(a0, t_begin + w);
-    for (int t0 = t_begin + w; t0 < n16; t0 += 8 * kBatch) {
-      if (t0 + 4 * kBatch < n16) load_a(a1, t0 + 4 * kBatch);
+    for (int t0 = t_begin + w; t0 < n32; t0 += 2 * kStep) {
+      if (t0 + kStep < n32) load_a(a1, t0 + kStep);
       issue_here();
       out_tiles(a0, t0);
-      if (t0 + 4 * kBatch < n16) {
-        if (t0 + 8 * kBatch < n16) load_a(a0, t0 + 8 * kBatch);
+      if (t0 + kStep < n32) {
+        if (t0 + 2 * kStep < n32) load_a(a0, t0 + 2 * kStep);
         issue_here();
-        out_tiles(a1, t0 + 4 * kBatch);
+        out_tiles(a1, t0 + kStep);
       }
     }
   }
@@ -543,16 +574,15 @@ __global__ __launch_bounds__(kThreads) void lora_bwd_rows_kernel(
 //   dBq[j][i] = fp16(sum_m gs_q[m][j] t[m][i])        j < NQ, i < r,  gs_x = fp16(g_x * s)
 //   dBv[j][i] = fp16(sum_m gs_v[m][j] t[m][r + i])    j < NV, i < r
 // each cast to fp32 (the fp16 GEMM result cast to the fp32 parameter, as autocast's backward
-// gives it).  lora_params_partial_kernel: workgroup (column block of 64, slice of kSlice rows)
+// gives it).  lora_params_partial_kernel: workgroup (column block of 64, slice of rows)
 // stages 64-row chunks of X (y, or g_q / g_v scaled and rounded to gs as they are staged: its
 // 64 columns) and Z (dt or t) through LDS,
 // transposed so that each MFMA operand is 8 consecutive rows of one column, and writes fp32
 // partial sums per slice; lora_params_reduce_kernel adds the slices in order and rounds.
 // With the next chunk's loads issued before the current chunk's MFMAs and the reduce's loads
 // issued eight slices at a time, the pair took 10.5 us against 13.2 us at 2048 rows on
-// MI355X (identical bits); 256-row slices were faster at 2048 rows (9.4 us) but slower at 888
-// (8.0 against 7.3 us), 64-row slices slower at both.
-constexpr int kSlice = 128;        // rows per slice
+// MI355X (identical bits).  The slices grow with the rows (params_slice).
+constexpr int kSlice = 128;        // rows of the smallest slice
 constexpr int kChunk = 64;         // rows per LDS chunk
 constexpr int kPStride = kChunk + 8;   // transposed tile row (halves): 144 B, 16-B aligned
 
@@ -587,7 +617,7 @@ __global__ __launch_bounds__(kThreads) void lora_params_partial_kernel(
     const uint16_t* __restrict__ y, const uint16_t* __restrict__ t,
     const uint16_t* __restrict__ dt, const uint16_t* __restrict__ gq, int64_t ldq,
     const uint16_t* __restrict__ gv, int64_t ldv, float scaling, float* __restrict__ part, int M,
-    int H, int NQ, int NV, int64_t n_out) {
+    int H, int NQ, int NV, int64_t n_out, int slice_rows) {
   __shared__ __align__(16) _Float16 XT[64 * kPStride];       // [64 columns][64 rows]
   __shared__ __align__(16) _Float16 ZT[2 * kR * kPStride];   // [32 columns][64 rows]
   const int nba = H / 64, nbq = NQ / 64;
@@ -601,7 +631,7 @@ __global__ __launch_bounds__(kThreads) void lora_params_partial_kernel(
   const uint16_t* Z = (kind == 0 ? dt : t) + (kind == 2 ? kR : 0);
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int ql = lane & 15, gr = lane >> 4;
-  const int r_begin = slice * kSlice, r_end = min(M, r_begin + kSlice);
+  const int r_begin = slice * slice_rows, r_end = min(M, r_begin + slice_rows);
   // dA: C = X^T Z tiles (row = X column, column = Z column): wave w owns X columns 16w..+15
   //     and both Z tiles; dB: C = Z^T X (row = Z column, column = X column): wave w owns X
   //     columns 16w..+15.  Either way a lane's 4 results are 4 consecutive partial entries.
@@ -692,15 +722,19 @@ int check_dims(int64_t M, int32_t H, int32_t NQ, int32_t NV, int32_t r) {
 
 bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) != 0; }
 
-// Column parts per row block: about kTargetGroups workgroups in all, each part at least
-// 4 * kBatch output tiles (one batch per wavefront).
+// Column parts per row block: at most kTargetGroups workgroups in all (one a CU) while the row
+// blocks alone do not fill the GPU, each part at least 4 * kBatch output tiles (one batch per
+// wavefront).  Every workgroup is one serial chain (the rank-2r product, then its tiles) that
+// keeps its CU's loads busy, so a second one on some of the CUs doubles the time: rounding the
+// parts up (280 workgroups at 888 rows) measured 15.1 us for the RoPE form and 10.9 for the row
+// backward, rounded down 10.2 and 7.7; at 2100 rows 19.3 and 12.6 against 16.1 and 10.6.
 #ifndef SOUPK_LORA_TARGET_GROUPS
 #define SOUPK_LORA_TARGET_GROUPS 256
 #endif
 constexpr int64_t kTargetGroups = SOUPK_LORA_TARGET_GROUPS;
 unsigned column_parts(int64_t M, int n_tiles) {
   const int64_t row_blocks = (M + kRows - 1) / kRows;
-  int64_t parts = (kTargetGroups + row_blocks - 1) / row_blocks;
+    int64_t parts = kTargetGroups / row_blocks;
   parts = std::min<int64_t>(parts, std::max(1, n_tiles / (4 * kBatch)));
   return static_cast<unsigned>(std::max<int64_t>(parts, 1));
 }
@@ -800,6 +834,17 @@ static int64_t lora_params_workspace(int64_t M, int32_t H, int32_t NQ, int32_t N
 
 namespace {
 
+// Rows per slice: kSlice while that gives fewer than two dozen slices, then the power of two
+// that leaves 12 to 23 of them, so that the partial sums (312 KB a slice) written and read back
+// stop growing with the rows.  Measured with 128- / 256- / 512-row slices: 888 rows 8.0 / 9.4 /
+// 12.9 us, 2048 rows 10.9 / 10.4 / 13.7, 4096 rows 16.2 / 13.8 / 15.6, 8192 rows 28.5 / 25.1 /
+// 22.0.
+int params_slice(int64_t M) {
+  int64_t rows = kSlice;
+  while (M / (2 * rows) >= 12) rows *= 2;
+  return static_cast<int>(rows);
+}
+
 // The two launches of the parameter gradients over a caller-given partial-sum buffer `part`
 // (at least lora_params_workspace(M, H, NQ, NV) floats).  The partial kernel writes every
 // entry of every slice, so `part` needs no clearing and its old contents never leak into a
@@ -815,11 +860,12 @@ int lora_params_launch(const uint16_t* y, const uint16_t* t, const uint16_t* dt,
     return launch_kernel(lora_params_reduce_kernel, dim3(reduce_grid), dim3(256), st,
                          static_cast<const float*>(nullptr), 0, n_out, H, NQ, d_aq, d_av,
                          d_bq, d_bv);
-  const int slices = static_cast<int>((M + kSlice - 1) / kSlice);
+  const int slice_rows = params_slice(M);
+  const int slices = static_cast<int>((M + slice_rows - 1) / slice_rows);
   const dim3 grid(static_cast<unsigned>(H / 64 + NQ / 64 + NV / 64),
                   static_cast<unsigned>(slices));
   int rc2 = launch_kernel(lora_params_partial_kernel, grid, dim3(kThreads), st, y, t, dt, g_q,
-                          ld_q, g_v, ld_v, scaling, part, static_cast<int>(M), H, NQ, NV, n_out);
+                          ld_q, g_v, ld_v, scaling, part, static_cast<int>(M), H, NQ, NV, n_out, slice_rows);
   if (rc2 != kOk) return rc2;
   return launch_kernel(lora_params_reduce_kernel, dim3(reduce_grid), dim3(256), st, part,
                        slices, n_out, H, NQ, d_aq, d_av, d_bq, d_bv);
