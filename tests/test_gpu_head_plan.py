@@ -100,3 +100,44 @@ def test_no_synchronisation_under_capture():
         for a, b in zip(outs, want):
             assert torch.equal(a, b)
         assert torch.equal(dx, dy)
+
+
+def test_planned_gradient_batched_and_differentiated():
+    """Several loss gradients at once (is_grads_batched) and a gradient of the gradient: each equal
+    to what the general form gives, as the same products of one fp16 row and one fp32 factor."""
+    h, w, t = _inputs(40, 64, 5000, 0.4, 11)
+    x = h.clone().requires_grad_(True)
+    loss = head.fused_head_loss(x, w, t, torch.tensor(24, device=DEV))[0]
+    one = torch.autograd.grad(loss, x, torch.tensor(2048.0, device=DEV), retain_graph=True)[0]
+    many = torch.autograd.grad(loss, x, torch.tensor([1024.0, 2048.0], device=DEV),
+                               is_grads_batched=True, retain_graph=True)[0]
+    assert many.shape == (2, 40, 64) and torch.equal(many[1], one)
+    s = torch.tensor(2048.0, device=DEV, requires_grad=True)
+    dh = torch.autograd.grad(loss, x, s, create_graph=True)[0]
+    assert torch.equal(dh, one)
+    # d(sum dh)/ds = sum dh / s, fp16 rounding of each entry of dh apart
+    ds = torch.autograd.grad(dh.float().sum(), s)[0]
+    want = float(one.double().sum()) / 2048.0
+    bound = 2.0 ** -10 * float(one.double().abs().sum()) / 2048.0
+    assert abs(float(ds) - want) <= bound
+
+
+def test_refusals_stay():
+    """Targets of another shape, an autocast to another type and a denominator that is no number
+    are refused as by the general form."""
+    h, w, t = _inputs(8, 64, 5000, 0.0, 12)
+    with pytest.raises(ValueError):
+        head.fused_head_loss(h, w, t.view(2, 4), 8)
+    with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(TypeError):
+        head.fused_head_loss(h, w, t, 8)
+    with pytest.raises(ValueError):
+        head.fused_head_loss(h, w, t, float("nan"))
+
+
+def test_wrapped_tensors_raise():
+    """A batched tensor has no storage to hand to a kernel: an error, as an exception."""
+    from testt_amd import mlp
+
+    gu = torch.zeros(3, 4, 64, dtype=torch.float16, device=DEV)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(mlp.gated_silu)(gu)

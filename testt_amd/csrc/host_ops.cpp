@@ -153,13 +153,27 @@ Tensor empty(at::IntArrayRef size, at::ScalarType dt, const at::Device& dev) {
 PyObject* g_error = nullptr;        // testt_amd._ext.SoupkError
 const char* (*p_status_string)(int) = nullptr;
 
+// The GIL given up for a scope, taken back also when an exception leaves it: a tensor without a
+// storage (a functorch wrapper, for one) throws from data_ptr, and HANDLE_TH_ERRORS sets the Python
+// error from it.
+class NoGil {
+ public:
+  NoGil() : state_(PyEval_SaveThread()) {}
+  ~NoGil() { PyEval_RestoreThread(state_); }
+  NoGil(const NoGil&) = delete;
+  NoGil& operator=(const NoGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
 // The launch's status as the Python layer reports it; true when it succeeded.
 template <class F>
 bool launched(const char* name, F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
+  const int rc = [&] {
+    const NoGil released;
+    return f();
+  }();
   if (rc == 0) return true;
   const char* text = p_status_string ? p_status_string(rc) : nullptr;
   PyErr_Format(g_error ? g_error : PyExc_RuntimeError, "%s failed with status %d: %s", name, rc,

@@ -172,7 +172,10 @@ def _denominator_args(denominator, device):
 def _device_plan(hidden, weight, denominator):
     """The arguments of the forward without a host synchronisation, or None where the general
     form runs: fp16 rows and head on one device, a vocabulary whose rows are whole 16-byte chunks
-    (the gradient rows keep the logits rows' alignment) and operands gemm_nn takes."""
+    (the gradient rows keep the logits rows' alignment) and operands gemm_nn takes.  An autocast
+    to another type stays with the general form, which refuses the logits that it makes."""
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
+        return None
     rows, width = hidden.shape
     vocab = weight.shape[0]
     if rows == 0 or not hidden.is_cuda or hidden.dtype != torch.float16 or \
@@ -197,9 +200,9 @@ def _forward_device(ctx, hidden, weight, targets, den):
     correct = torch.empty(rows, dtype=torch.int32, device=dev)
     want_grad = ctx.needs_input_grad[0]
     slot = packed = scal = None
+    unit = _grad_unit(den_host) if den_ptr is None else 0.0   # (refuses a denominator of inf or nan)
+    scale = unit / max(den_host, 1e-6)
     if want_grad:
-        unit = _grad_unit(den_host) if den_ptr is None else 0.0
-        scale = unit / max(den_host, 1e-6)
         slot = torch.empty(rows, dtype=torch.int32, device=dev)
         counts = torch.empty(-(-rows // chunk), dtype=torch.int32, device=dev)
         scal = torch.empty(2, dtype=torch.float32, device=dev)
@@ -234,6 +237,16 @@ def _forward_device(ctx, hidden, weight, targets, den):
     return (loss, *stats)
 
 
+def _planned_hidden_grad(packed, slot, scal, chunk, grad_loss):
+    """soupk_head_dh in torch operations, for a loss gradient that is batched (vmap) or itself
+    differentiated."""
+    at = torch.arange(slot.numel(), device=slot.device)
+    at = at - at % chunk + slot.clamp(min=0)
+    rows = torch.where((slot >= 0)[:, None], packed.index_select(0, at), 0)
+    factor = grad_loss / scal[1]
+    return (rows.to(torch.float32) * factor).to(torch.float16)
+
+
 class FusedHeadLoss(torch.autograd.Function):
     """(loss, entropy [M], token loss [M], correct [M]) of the frozen head over `hidden`
     (solution/head.py:87-137's interface); the gradient for `hidden` is computed in forward."""
@@ -244,6 +257,8 @@ class FusedHeadLoss(torch.autograd.Function):
         vocab = weight.shape[0]
         dev = hidden.device
         targets = targets.to(torch.int64).contiguous()
+        if targets.dim() != 1:
+            raise ValueError(f"targets must have 1 dim, got shape {tuple(targets.shape)}")
         den = _device_plan(hidden, weight, denominator)
         if den is not None and targets.device == dev and targets.numel() == rows:
             return _forward_device(ctx, hidden.contiguous(), weight, targets, den)
@@ -304,8 +319,15 @@ class FusedHeadLoss(torch.autograd.Function):
         if ctx.planned:
             packed, slot, scal = ctx.saved_tensors
             grad_loss = grad_loss.to(torch.float32).contiguous()
+            try:
+                address = None if torch.is_grad_enabled() else grad_loss.data_ptr()
+            except RuntimeError:        # (a batched tensor has no storage)
+                address = None
+            if address is None:
+                dh = _planned_hidden_grad(packed, slot, scal, ctx.chunk, grad_loss)
+                return dh, None, None, None
             dh = torch.empty_like(packed)
-            _ext.call("soupk_head_dh", packed.data_ptr(), slot.data_ptr(), grad_loss.data_ptr(),
+            _ext.call("soupk_head_dh", packed.data_ptr(), slot.data_ptr(), address,
                       scal.data_ptr(), dh.data_ptr(), packed.shape[0], packed.shape[1], ctx.chunk,
                       _ext.stream_of(dh))
             return dh, None, None, None
