@@ -379,3 +379,35 @@ def test_nf4_resident_native_is_bit_identical(monkeypatch, lengths, with_delta):
     names = ["s", "d", "d s_in", "d delta"] * 2 + ["d A_q", "d B_q", "d A_v", "d B_v"]
     for name, a, b in zip(names, *runs):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("lengths", [(64, 37), (31, 32), (1, 0)])
+def test_nf4_resident_layer_native_is_bit_identical(monkeypatch, lengths):
+    """The layer on its NF4 weights issued from C, where the q|k|v input gradient is added to the
+    LoRA part by the kernel that sums the contraction's parts, against the same layer issued from
+    Python, which adds it by an operation of its own: the same values, bit for bit."""
+    print(f"nf4-resident layer native lengths={lengths}", flush=True)
+    batch, seq = len(lengths), 64
+    w = layer.synthetic_layer(DEV, seed=15)
+    amask = torch.zeros(batch, seq, dtype=torch.int64, device=DEV)
+    for b, n in enumerate(lengths):
+        amask[b, :n] = 1
+    pos = amask.reshape(-1).nonzero().squeeze(1)
+    m = pos.numel()
+    cos, sin = (t.to(DEV) for t in workloads.rope_tables(seq, w.head_dim))
+    g = torch.Generator().manual_seed(9)
+    s0 = torch.randn(m, workloads.HIDDEN, generator=g).to(DEV)
+    d0 = (0.5 * torch.randn(m, workloads.HIDDEN, generator=g)).to(torch.float16).to(DEV)
+    gs = (1e-2 * torch.randn(m, workloads.HIDDEN, generator=g)).to(DEV)
+    gd = (1e-2 * torch.randn(m, workloads.HIDDEN, generator=g)).to(torch.float16).to(DEV)
+    runs = []
+    for native in (True, False):
+        monkeypatch.setattr(layer_native, "NATIVE_LAYER", native)
+        s_in, d_in = s0.clone().requires_grad_(True), d0.clone().requires_grad_(True)
+        s, d = layer.decoder_layer(s_in, d_in, w, pos, batch, seq, cos, sin,
+                                   layer.key_valid_of(amask))
+        leaves = [s_in, d_in, *w.lora_q, *w.lora_v]
+        runs.append([s.detach(), d.detach(), *torch.autograd.grad([s, d], leaves, [gs, gd])])
+    for name, a, b in zip(["s", "d", "d s_in", "d delta", "d A_q", "d B_q", "d A_v", "d B_v"],
+                          *runs):
+        assert torch.equal(a, b), name

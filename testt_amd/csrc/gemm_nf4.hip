@@ -634,12 +634,16 @@ constexpr int kMaxSplits = 32;
 // y = fp16(((p[0] + p[1]) + ...) + bias) over the splits' fp32 partials [splits, M, N], four
 // consecutive outputs per thread (N is a multiple of 64), partials added in split order.  All
 // of a thread's loads are issued before the first add (unrolled to kMaxSplits under a uniform
-// test), so the kernel waits on memory once, not once per split.
+// test), so the kernel waits on memory once, not once per split.  With `add` (which may be y
+// itself) the rounded sum is added to it, the total in fp32 and rounded again: the values of a
+// separate fp16 addition without its launch and its pass.
 __global__ __launch_bounds__(256) void split_sum_kernel(
     const f32x4* __restrict__ parts, int splits, int64_t stride4, int64_t n4, int n_cols4,
-    const uint16_t* __restrict__ bias, u32x2* __restrict__ y) {
+    const uint16_t* __restrict__ bias, const u32x2* add, u32x2* y) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= n4) return;
+  u32x2 a = {0u, 0u};
+  if (add != nullptr) a = add[i];
   f32x4 v[kMaxSplits];
 #pragma unroll
   for (int p = 0; p < kMaxSplits; ++p)
@@ -653,7 +657,11 @@ __global__ __launch_bounds__(256) void split_sum_kernel(
     const u32x2 bw = *reinterpret_cast<const u32x2*>(bias + c);
     s = s + f32x4{lo_h(bw.x), hi_h(bw.x), lo_h(bw.y), hi_h(bw.y)};
   }
-  y[i] = u32x2{pack_h2(s[0], s[1]), pack_h2(s[2], s[3])};
+  u32x2 out = {pack_h2(s[0], s[1]), pack_h2(s[2], s[3])};
+  if (add != nullptr)
+    out = u32x2{pack_h2(lo_h(a.x) + lo_h(out.x), hi_h(a.x) + hi_h(out.x)),
+                pack_h2(lo_h(a.y) + lo_h(out.y), hi_h(a.y) + hi_h(out.y))};
+  y[i] = out;
 }
 
 // Contraction steps per split and the splits that leaves non-empty, for `kt` 64-wide steps cut
@@ -666,6 +674,15 @@ int split_plan(int kt, int32_t splits, int& per, int& used) {
 }
 
 }  // namespace
+
+// soupk_gemm_nn_nf4_split with dx = add + the product where `add` is given (layer_exec.hip)
+__attribute__((visibility("hidden"))) int gemm_nn_nf4_split_add(
+    const uint16_t* dy, int64_t lddy, int32_t n_parts, const uint8_t* const* packed,
+    const uint8_t* const* absmax_u8, const float* const* code2, const float* const* absmax2,
+    const float* const* offset, const float* const* nf4, const int32_t* part_rows,
+    int32_t qblock, int32_t qblock2, const uint16_t* add, uint16_t* dx, int64_t M, int32_t N,
+    int32_t K, int32_t splits, float* workspace, int64_t workspace_floats, void* stream);
+
 }  // namespace soupk
 
 using namespace soupk;
@@ -764,7 +781,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_tn_nf4_split(
   return launch_kernel(split_sum_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)),
                        dim3(256), st, reinterpret_cast<const f32x4*>(workspace), used,
                        M * static_cast<int64_t>(N) / 4, n4, N / 4, bias,
-                       reinterpret_cast<u32x2*>(y));
+                       static_cast<const u32x2*>(nullptr), reinterpret_cast<u32x2*>(y));
 }
 
 namespace {
@@ -837,11 +854,11 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4(
                        N, K, nullptr, K / 64);
 }
 
-extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4_split(
+int soupk::gemm_nn_nf4_split_add(
     const uint16_t* dy, int64_t lddy, int32_t n_parts, const uint8_t* const* packed,
     const uint8_t* const* absmax_u8, const float* const* code2, const float* const* absmax2,
     const float* const* offset, const float* const* nf4, const int32_t* part_rows,
-    int32_t qblock, int32_t qblock2, uint16_t* dx, int64_t M, int32_t N, int32_t K,
+    int32_t qblock, int32_t qblock2, const uint16_t* add, uint16_t* dx, int64_t M, int32_t N, int32_t K,
     int32_t splits, float* workspace, int64_t workspace_floats, void* stream) {
   Nf4Weights nw;
   const int rc = check_nn(dy, lddy, n_parts, packed, absmax_u8, code2, absmax2, offset, nf4,
@@ -852,6 +869,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4_split(
   if (workspace_floats < static_cast<int64_t>(used) * M * N) return kInvalid;
   if (M == 0) return kOk;
   if (bad_ptr(dy) || bad_ptr(dx) || bad_ptr(workspace)) return kInvalid;
+  if (reinterpret_cast<uintptr_t>(add) & 7) return kInvalid;   // read 4 halves at a time
   hipStream_t st = static_cast<hipStream_t>(stream);
   int r;
   if (M <= kNnSmallRows)
@@ -874,5 +892,17 @@ extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4_split(
   const int64_t n4 = M * static_cast<int64_t>(N) / 4;
   return launch_kernel(split_sum_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)),
                        dim3(256), st, reinterpret_cast<const f32x4*>(workspace), used, n4, n4,
-                       N / 4, nullptr, reinterpret_cast<u32x2*>(dx));
+                       N / 4, nullptr, reinterpret_cast<const u32x2*>(add),
+                       reinterpret_cast<u32x2*>(dx));
+}
+
+extern "C" __attribute__((visibility("default"))) int soupk_gemm_nn_nf4_split(
+    const uint16_t* dy, int64_t lddy, int32_t n_parts, const uint8_t* const* packed,
+    const uint8_t* const* absmax_u8, const float* const* code2, const float* const* absmax2,
+    const float* const* offset, const float* const* nf4, const int32_t* part_rows,
+    int32_t qblock, int32_t qblock2, uint16_t* dx, int64_t M, int32_t N, int32_t K,
+    int32_t splits, float* workspace, int64_t workspace_floats, void* stream) {
+  return gemm_nn_nf4_split_add(dy, lddy, n_parts, packed, absmax_u8, code2, absmax2, offset, nf4,
+                               part_rows, qblock, qblock2, nullptr, dx, M, N, K, splits, workspace,
+                               workspace_floats, stream);
 }

@@ -734,7 +734,7 @@ bool misaligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) !=
 constexpr int64_t kTargetGroups = SOUPK_LORA_TARGET_GROUPS;
 unsigned column_parts(int64_t M, int n_tiles) {
   const int64_t row_blocks = (M + kRows - 1) / kRows;
-    int64_t parts = kTargetGroups / row_blocks;
+  int64_t parts = kTargetGroups / row_blocks;
   parts = std::min<int64_t>(parts, std::max(1, n_tiles / (4 * kBatch)));
   return static_cast<unsigned>(std::max<int64_t>(parts, 1));
 }
