@@ -598,9 +598,10 @@ OP(gemm) {
   END_HANDLE_TH_ERRORS
 }
 
-// nf4_key(weight) -> bytes: what a plan of an NF4 weight depends on, the addresses of its packed data
-// and state tensors, their device, the offset object, the shape and the block size; None for an
-// object without that state.
+// nf4_key(weight) -> bytes: everything a plan of an NF4 weight is made from and checked on -- for the
+// packed data and each state tensor its address, element count, type, device and whether it is
+// contiguous; the same of the offset, or its value when it is a number; the shape; both block sizes;
+// whether it is nested NF4.  None for an object without that state.
 struct Ref {
   PyObject* o;
   ~Ref() { Py_XDECREF(o); }
@@ -613,8 +614,9 @@ OP(nf4_key) {
       PyUnicode_InternFromString("quant_state"), PyUnicode_InternFromString("data"),
       PyUnicode_InternFromString("absmax"),      PyUnicode_InternFromString("code"),
       PyUnicode_InternFromString("state2"),      PyUnicode_InternFromString("offset"),
-      PyUnicode_InternFromString("shape"),       PyUnicode_InternFromString("blocksize")};
-  auto get = [](PyObject* o, int i) { return Ref{PyObject_GetAttr(o, names[i])}; };
+      PyUnicode_InternFromString("shape"),       PyUnicode_InternFromString("blocksize"),
+      PyUnicode_InternFromString("quant_type"),  PyUnicode_InternFromString("nested")};
+  auto get = [](PyObject* o, int i) { return Ref{o ? PyObject_GetAttr(o, names[i]) : nullptr}; };
   const Ref state = get(a[0], 0);
   if (!state.o) {
     PyErr_Clear();
@@ -622,35 +624,55 @@ OP(nf4_key) {
   }
   const Ref data = get(a[0], 1), absmax = get(state.o, 2), code = get(state.o, 3),
             state2 = get(state.o, 4), offset = get(state.o, 5), shape = get(state.o, 6),
-            block = get(state.o, 7);
-  const Ref code2{state2.o ? PyObject_GetAttr(state2.o, names[3]) : nullptr},
-      absmax2{state2.o ? PyObject_GetAttr(state2.o, names[2]) : nullptr};
+            block = get(state.o, 7), type = get(state.o, 8), nested = get(state.o, 9);
+  const Ref code2 = get(state2.o, 3), absmax2 = get(state2.o, 2), block2 = get(state2.o, 7);
   if (PyErr_Occurred()) {
     PyErr_Clear();
     ELSE_PYTHON;
   }
-  uintptr_t key[10];
+  uint64_t key[24];
   int i = 0;
+  auto tensor = [&](PyObject* o) {
+    const Tensor& t = THPVariable_Unpack(o);
+    const at::Device d = t.device();
+    key[i++] = reinterpret_cast<uintptr_t>(t.data_ptr());
+    key[i++] = static_cast<uint64_t>(t.numel());
+    key[i++] = static_cast<uint64_t>(static_cast<uint8_t>(t.scalar_type())) |
+               static_cast<uint64_t>(t.is_contiguous()) << 8 |
+               static_cast<uint64_t>(static_cast<uint8_t>(d.type())) << 16 |
+               static_cast<uint64_t>(static_cast<uint8_t>(d.index())) << 24;
+  };
   for (PyObject* o : {data.o, absmax.o, code.o, code2.o, absmax2.o}) {
-    if (!o || !THPVariable_Check(o)) ELSE_PYTHON;
-    key[i++] = reinterpret_cast<uintptr_t>(THPVariable_Unpack(o).data_ptr());
+    if (!THPVariable_Check(o)) ELSE_PYTHON;
+    tensor(o);
   }
-  key[i++] = static_cast<uintptr_t>(THPVariable_Unpack(data.o).get_device());
-  key[i++] = reinterpret_cast<uintptr_t>(offset.o);
+  if (THPVariable_Check(offset.o)) {
+    tensor(offset.o);
+  } else {
+    const double v = PyFloat_AsDouble(offset.o);
+    std::memcpy(&key[i++], &v, sizeof(v));
+    key[i++] = ~uint64_t{0};               // (no tensor)
+    key[i++] = ~uint64_t{0};
+  }
   if (PySequence_Size(shape.o) != 2) {
     PyErr_Clear();
     ELSE_PYTHON;
   }
   for (Py_ssize_t d = 0; d < 2; ++d) {
     const Ref n{PySequence_GetItem(shape.o, d)};
-    key[i++] = n.o ? static_cast<uintptr_t>(PyLong_AsUnsignedLongLongMask(n.o)) : 0;
+    key[i++] = n.o ? PyLong_AsUnsignedLongLongMask(n.o) : 0;
   }
-  key[i] = static_cast<uintptr_t>(PyLong_AsUnsignedLongLongMask(block.o));
+  key[i++] = PyLong_AsUnsignedLongLongMask(block.o);
+  key[i++] = PyLong_AsUnsignedLongLongMask(block2.o);
+  const int is_nested = PyObject_IsTrue(nested.o);
+  key[i++] = (is_nested == 1 ? 1u : 0u) |
+             (PyUnicode_Check(type.o) && !PyUnicode_CompareWithASCIIString(type.o, "nf4") ? 2u : 0u);
   if (PyErr_Occurred()) {
     PyErr_Clear();
     ELSE_PYTHON;
   }
-  return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof(key));
+  static_assert(sizeof(key) >= (6 * 3 + 2 + 3) * sizeof(key[0]));
+  return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), i * sizeof(key[0]));
   END_HANDLE_TH_ERRORS
 }
 

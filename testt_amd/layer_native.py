@@ -123,9 +123,8 @@ def _nf4_group(weights, dev):
 def _nf4_layer(w, M, dev):
     """The LayerNf4 of a layer's NF4 weights at M tokens: the split counts nf4_gemm's
     nf4_linear and nf4_grad_input pick, and the floats of the largest split's partials
-    (partials unset).  Remembered on the q weight per token count, device and weight state (the
-    addresses of the seven weights' NF4 data and tables, as nf4's plan cache keys them), so
-    that it lives as long as the weights whose tables it points at; a fresh copy of the
+    (partials unset).  Remembered on the q weight per token count, device and weight state (as
+    nf4's plan cache keys it), with the plans whose tables it points at; a fresh copy of the
     remembered struct per call."""
     from . import nf4
 
@@ -140,7 +139,7 @@ def _nf4_layer(w, M, dev):
         if len(memo) > 64:
             memo.clear()
         n4, fwd, bwd = _build_nf4_layer(w, M, dev)
-        hit = memo[key] = (bytes(n4), fwd, bwd)
+        hit = memo[key] = (bytes(n4), fwd, bwd, [nf4._plan(x, dev) for x in weights])
     return LayerNf4.from_buffer_copy(hit[0]), hit[1], hit[2]
 
 

@@ -103,9 +103,9 @@ def _f32(t):
 
 
 def _plan_key(weight, device):
-    """What a cached plan of `weight` depends on: the addresses of its packed data and state
-    tensors, the offset object, the shape and the block size (None for an object that is not an
-    NF4 weight)."""
+    """What a cached plan of `weight` was made from and checked on (host_ops.cpp's nf4_key): address,
+    size, type, device and layout of its packed data, state tensors and offset, its shape, block
+    sizes and format (None for an object that is not an NF4 weight)."""
     key = _ext.host().nf4_key(weight)
     return None if key is None else (device, key)
 
@@ -113,8 +113,9 @@ def _plan_key(weight, device):
 def _plan(weight, device):
     """The kernel arguments of one weight on `device` (pointers into its quant state, converted
     tables kept alive), checked once and cached on the weight; None for a layout or device the
-    kernel does not take.  The cache is keyed by the addresses of the state tensors, so a
-    weight whose state is replaced is checked again."""
+    kernel does not take.  The cache is keyed by all that is checked here (_plan_key), so a
+    weight whose state is replaced is checked again; the state tensors are kept with the plan,
+    so that no other tensor can come to lie at an address of the key while it is in use."""
     key = _plan_key(weight, device)
     if key is None:
         return None
@@ -139,7 +140,9 @@ def _plan(weight, device):
     offset = _offset_tensor(state, device)
     plan = ((_ext.ptr(weight.data), _ext.ptr(absmax), _ext.ptr(code2), _ext.ptr(absmax2),
              _ext.ptr(offset), _ext.ptr(nf4)), n_bytes, int(state.blocksize),
-            int(state.state2.blocksize), (absmax, code2, absmax2, nf4, offset))
+            int(state.state2.blocksize),
+            (absmax, code2, absmax2, nf4, offset,
+             (state.absmax, state.state2.code, state.state2.absmax, state.code, state.offset)))
     try:
         weight._soupk_plan = (key, plan)
     except AttributeError:          # objects without a __dict__ are checked on every call
