@@ -130,10 +130,10 @@ def _nf4_layer(w, M, dev):
 
     weights = (w.q, w.k, w.v, w.o, w.gate, w.up, w.down)
     key = (M, dev, tuple(nf4._plan_key(x, dev) for x in weights))
-    memo = getattr(w.q, "_soupk_layer_nf4", None)
+    memo = nf4.Kept.of(w.q, "_soupk_layer_nf4", None)
     if memo is None:
         memo = {}
-        setattr(w.q, "_soupk_layer_nf4", memo)
+        nf4.Kept.put(w.q, "_soupk_layer_nf4", None, memo)
     hit = memo.get(key)
     if hit is None:
         if len(memo) > 64:

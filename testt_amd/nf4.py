@@ -110,6 +110,33 @@ def _plan_key(weight, device):
     return None if key is None else (device, key)
 
 
+class Kept:
+    """What a call prepared for a weight, kept on it as an attribute: addresses, which mean nothing to
+    a copy of the weight or to another process.  A copy or pickle of the weight holds an empty
+    tuple in its place and prepares its own."""
+
+    __slots__ = ("key", "value")
+
+    def __init__(self, key, value):
+        self.key, self.value = key, value
+
+    def __reduce__(self):
+        return tuple, ()
+
+    @classmethod
+    def of(cls, weight, name, key):
+        """What is kept on `weight` under `name` for `key`; None for another key, or nothing kept."""
+        kept = getattr(weight, name, None)
+        return kept.value if type(kept) is cls and kept.key == key else None
+
+    @classmethod
+    def put(cls, weight, name, key, value):
+        try:
+            setattr(weight, name, cls(key, value))
+        except AttributeError:          # an object without a __dict__: prepared on every call
+            pass
+
+
 def _plan(weight, device):
     """The kernel arguments of one weight on `device` (pointers into its quant state, converted
     tables kept alive), checked once and cached on the weight; None for a layout or device the
@@ -120,9 +147,9 @@ def _plan(weight, device):
     if key is None:
         return None
     state = _quant_state(weight)
-    cached = getattr(weight, "_soupk_plan", None)
-    if cached is not None and cached[0] == key:
-        return cached[1]
+    cached = Kept.of(weight, "_soupk_plan", key)
+    if cached is not None:
+        return cached
     if not (supports_fast_unpack(weight) and _on_device(weight, device)):
         return None
     if state.absmax.dtype != torch.uint8:
@@ -143,10 +170,7 @@ def _plan(weight, device):
             int(state.state2.blocksize),
             (absmax, code2, absmax2, nf4, offset,
              (state.absmax, state.state2.code, state.state2.absmax, state.code, state.offset)))
-    try:
-        weight._soupk_plan = (key, plan)
-    except AttributeError:          # objects without a __dict__ are checked on every call
-        pass
+    Kept.put(weight, "_soupk_plan", key, plan)
     return plan
 
 
@@ -256,6 +280,9 @@ class _GroupPlan:
     the same device, the same grouping and the same weights (by identity), each with an
     unchanged plan key (its packed data and state tensors, _plan_key)."""
 
+    def __reduce__(self):           # (left out of copies and pickles, as Kept)
+        return tuple, ()
+
     def __init__(self, device, sizes, flat_w, offsets, stacks, total):
         plans = [_plan(w, device) for w in flat_w]
         self.ok = all(pl is not None for pl in plans) and len({(pl[2], pl[3]) for pl in plans}) == 1
@@ -318,7 +345,7 @@ class _GroupPlan:
 def _group_plan(groups, device, flat_w, offsets, stacks, total):
     sizes = tuple(len(g) for g in groups)
     plan = getattr(flat_w[0], "_soupk_groups", None)
-    if plan is None or not plan.matches(device, sizes, flat_w):
+    if type(plan) is not _GroupPlan or not plan.matches(device, sizes, flat_w):
         plan = _GroupPlan(device, sizes, flat_w, offsets, stacks, total)
         try:
             flat_w[0]._soupk_groups = plan

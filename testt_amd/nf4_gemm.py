@@ -58,15 +58,11 @@ def _stack(weights, device):
     keys = [_nf4._plan_key(w, device) for w in weights]
     if not keys or None in keys:
         return None
-    cached = getattr(weights[0], "_soupk_stack", None)
-    if cached is not None and cached[0] == keys:
-        return cached[1]
-    stack = _Stack(weights, device) if _readable(weights, device) else None
-    try:
-        weights[0]._soupk_stack = (keys, stack)
-    except AttributeError:          # objects without a __dict__ are checked on every call
-        pass
-    return stack
+    kept = _nf4.Kept.of(weights[0], "_soupk_stack", keys)
+    if kept is None:                # (a stack that the kernels do not read is kept as (None,))
+        kept = (_Stack(weights, device) if _readable(weights, device) else None,)
+        _nf4.Kept.put(weights[0], "_soupk_stack", keys, kept)
+    return kept[0]
 
 
 def _rows_fit(x, cols):
