@@ -82,20 +82,3 @@ def test_plan_keeps_no_weight_alive(stub_plans):
         assert first() is None
     finally:
         gc.enable()
-
-
-def test_groupings_keep_their_plans_side_by_side(stub_plans):
-    """A program that unpacks a layer's projections and, in between, the stack of one product."""
-    a, b, c = _Weight(8, 64), _Weight(4, 64), _Weight(4, 64)
-    layer, stack = [[a, b], [c]], [[a, b]]
-    p, q = _plan_for(layer), _plan_for(stack)
-    assert p is not q
-    for _ in range(2):
-        assert _plan_for(layer) is p and _plan_for(stack) is q
-
-
-def test_groupings_kept_are_bounded(stub_plans):
-    w = [_Weight(4, 64) for _ in range(3 * nf4._GROUPINGS_KEPT)]
-    for n in range(1, len(w) + 1):
-        _plan_for([w[:n]])
-        assert len(nf4.Kept.of(w[0], "_soupk_groups", None)) <= nf4._GROUPINGS_KEPT

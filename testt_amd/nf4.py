@@ -274,13 +274,14 @@ class _GroupPlan:
     arrays) and the byte offsets of the outputs; a call allocates the buffer and adds its
     address.
 
-    A plan is kept on the first weight of the list, one for each grouping (the number of weights
-    in each group; a later list of the same grouping that starts with the same weight replaces
-    it), so that the layer's seven projections and a single product's stack do not replace each
-    other.  It holds the weights only weakly, so it keeps no replaced weight
+    One plan is kept on the first weight of the list (a later list that starts with the same
+    weight replaces it).  It holds the weights only weakly, so it keeps no replaced weight
     alive and forms no reference cycle with the weight that carries it, and it is used only for
     the same device, the same grouping and the same weights (by identity), each with an
     unchanged plan key (its packed data and state tensors, _plan_key)."""
+
+    def __reduce__(self):           # (left out of copies and pickles, as Kept)
+        return tuple, ()
 
     def __init__(self, device, sizes, flat_w, offsets, stacks, total):
         plans = [_plan(w, device) for w in flat_w]
@@ -341,23 +342,15 @@ class _GroupPlan:
         return stacks, staged
 
 
-# Groupings whose plans one weight keeps at a time (a layer's seven projections; its q|k|v, gate|up
-# and single stacks where single products unpack; more only where a program regroups).
-_GROUPINGS_KEPT = 8
-
-
 def _group_plan(groups, device, flat_w, offsets, stacks, total):
     sizes = tuple(len(g) for g in groups)
-    plans = Kept.of(flat_w[0], "_soupk_groups", None)
-    if plans is None:
-        plans = {}
-        Kept.put(flat_w[0], "_soupk_groups", None, plans)
-    plan = plans.get(sizes)
-    if plan is None or not plan.matches(device, sizes, flat_w):
+    plan = getattr(flat_w[0], "_soupk_groups", None)
+    if type(plan) is not _GroupPlan or not plan.matches(device, sizes, flat_w):
         plan = _GroupPlan(device, sizes, flat_w, offsets, stacks, total)
-        if sizes not in plans and len(plans) >= _GROUPINGS_KEPT:
-            plans.clear()
-        plans[sizes] = plan
+        try:
+            flat_w[0]._soupk_groups = plan
+        except AttributeError:      # an object without a __dict__: planned on every call
+            pass
     return plan
 
 
