@@ -144,12 +144,15 @@ def _plan(weight, device):
     weight whose state is replaced is checked again; the state tensors are kept with the plan,
     so that no other tensor can come to lie at an address of the key while it is in use."""
     key = _plan_key(weight, device)
-    if key is None:
-        return None
-    state = _quant_state(weight)
+    return None if key is None else _plan_of(weight, device, key)
+
+
+def _plan_of(weight, device, key):
+    """_plan for a caller that has the weight's _plan_key."""
     cached = Kept.of(weight, "_soupk_plan", key)
     if cached is not None:
         return cached
+    state = _quant_state(weight)
     if not (supports_fast_unpack(weight) and _on_device(weight, device)):
         return None
     if state.absmax.dtype != torch.uint8:
@@ -172,6 +175,12 @@ def _plan(weight, device):
              (state.absmax, state.state2.code, state.state2.absmax, state.code, state.offset)))
     Kept.put(weight, "_soupk_plan", key, plan)
     return plan
+
+
+def _pointer_tables(ptrs):
+    """The plans' six pointers, one ctypes array over the weights for each (_plan's order)."""
+    table = ctypes.c_void_p * len(ptrs)
+    return [table(*column) for column in zip(*ptrs)]
 
 
 def unpack_into(weight, out):
@@ -229,7 +238,7 @@ def unpack_many(weights, outs):
         for c in range(0, len(items), MAX_PARTS_PER_LAUNCH):
             chunk = items[c:c + MAX_PARTS_PER_LAUNCH]
             n = len(chunk)
-            arrays = [(ctypes.c_void_p * n)(*[p[0][i] for p, _ in chunk]) for i in range(6)]
+            arrays = _pointer_tables([p[0] for p, _ in chunk])
             outs_a = (ctypes.c_void_p * n)(*[o.data_ptr() for _, o in chunk])
             sizes = (ctypes.c_int64 * n)(*[p[1] for p, _ in chunk])
             _ext.call("soupk_nf4_unpack_multi", n, *[ctypes.addressof(a) for a in arrays],
@@ -238,16 +247,31 @@ def unpack_many(weights, outs):
 
 
 def unpack_concat(weights, device):
-    """fp16 [sum N_i, K]: the weights stacked by rows, unpacked in place (one launch, its arguments
-    prepared once per list of weights: _GroupPlan)."""
-    device = torch.device(device)
-    if device.type == "cuda":
-        return unpack_groups((tuple(weights),), device)[0]
-    rows = [weight_shape(w)[0] for w in weights]
-    cols = weight_shape(weights[0])[1]
-    out = torch.empty((sum(rows), cols), dtype=torch.float16, device=device)
+    """fp16 [sum N_i, K]: the weights stacked by rows, unpacked in place by one launch where the kernel
+    takes them all.  Its arguments are put together on every call, from the weights' kept plans:
+    that takes no longer than to check a list of kept ones, costs nothing more on new weights, and
+    leaves the layer's plan of all its projections (_GroupPlan) where it is."""
+    shapes = [weight_shape(w) for w in weights]
+    cols = shapes[0][1]
+    out = torch.empty((sum([n for n, _ in shapes]), cols), dtype=torch.float16, device=device)
+    dev = out.device
+    plans = [_plan(w, dev) for w in weights] if kernels_ok(out) else [None]
+    if None not in plans and len(plans) <= MAX_PARTS_PER_LAUNCH and \
+            all([p[1:4] == (n * cols // 2, plans[0][2], plans[0][3])
+                 for p, (n, _) in zip(plans, shapes)]):
+        n = len(plans)
+        at, places = out.data_ptr(), []
+        for p in plans:
+            places.append(at)
+            at += 4 * p[1]                  # (two fp16 values for a packed byte)
+        arrays = _pointer_tables([p[0] for p in plans])
+        arrays.append((ctypes.c_void_p * n)(*places))
+        arrays.append((ctypes.c_int64 * n)(*[p[1] for p in plans]))
+        _ext.call("soupk_nf4_unpack_multi", n, *[ctypes.addressof(t) for t in arrays],
+                  plans[0][2], plans[0][3], _ext.stream_of(out))
+        return out
     views, start = [], 0
-    for n in rows:
+    for n, _ in shapes:
         views.append(out[start:start + n])
         start += n
     unpack_many(weights, views)
@@ -297,7 +321,7 @@ class _GroupPlan:
         for c in range(0, len(plans), MAX_PARTS_PER_LAUNCH):
             chunk = plans[c:c + MAX_PARTS_PER_LAUNCH]
             n = len(chunk)
-            arrays = [(ctypes.c_void_p * n)(*[pl[0][i] for pl in chunk]) for i in range(6)]
+            arrays = _pointer_tables([pl[0] for pl in chunk])
             sizes = (ctypes.c_int64 * n)(*[pl[1] for pl in chunk])
             self.launches.append((n, arrays, sizes, [2 * o for o in offsets[c:c + n]]))
 

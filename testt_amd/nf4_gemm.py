@@ -14,6 +14,7 @@ one split equals gemm_tn(x, unpack_concat(weights)) exactly; with more, the same
 summed in another order (fp32 partials per split, added in split order)."""
 
 import ctypes
+import threading
 
 import torch
 
@@ -24,32 +25,52 @@ MAX_PARTS = 4
 
 
 class _Stack:
-    """The launch arguments of one row stack of NF4 weights that the fused kernels read (1-4 parts
-    of one column count, each a multiple of 128 rows, blocksize 64, nested 256): the pointer tables
-    as ctypes arrays and their addresses in entry-point order."""
+    """One row stack of NF4 weights that the fused kernels read (1-4 parts of one column count, each
+    a multiple of 128 rows, blocksize 64, nested 256) and their launch arguments: the pointer
+    tables as ctypes arrays and their addresses in entry-point order, made at the first launch (a
+    stack that goes another way than through the fused kernels needs none)."""
 
-    def __init__(self, weights, device):
-        plans, rows, arrays, part_rows = _nf4_args(weights, device)
-        self.rows, self.cols = sum(rows), _nf4.weight_shape(weights[0])[1]
-        self.keep = (plans, arrays, part_rows)
-        self.args = (len(weights), *[ctypes.addressof(a) for a in arrays],
-                     ctypes.addressof(part_rows), plans[0][2], plans[0][3])
+    __slots__ = ("rows", "cols", "plans", "part_rows", "_args", "_keep")
+
+    def __init__(self, part_rows, cols, plans):
+        self.rows, self.cols = sum(part_rows), cols
+        self.plans, self.part_rows = plans, part_rows
+        self._args = None
+
+    @property
+    def args(self):
+        if self._args is None:
+            with _args_lock:            # (one set of arrays: the addresses are the arrays')
+                if self._args is None:
+                    n = len(self.plans)
+                    arrays = _nf4._pointer_tables([p[0] for p in self.plans])
+                    arrays.append((ctypes.c_int32 * n)(*self.part_rows))
+                    self._keep = arrays
+                    self._args = (n, *[ctypes.addressof(a) for a in arrays], self.plans[0][2],
+                                  self.plans[0][3])
+        return self._args
 
 
-def _readable(weights, device):
-    cols = None
+_args_lock = threading.Lock()
+
+
+def _make_stack(weights, device, keys):
+    """The _Stack of `weights`, whose plan keys are `keys`; None where the fused kernels do not read
+    them."""
     if not 1 <= len(weights) <= MAX_PARTS:
-        return False
-    for w in weights:
-        if not _nf4.supports_fast_unpack(w):
-            return False
-        st = w.quant_state
+        return None
+    cols, part_rows, plans = None, [], []
+    for w, key in zip(weights, keys):
         r, c = _nf4.weight_shape(w)
-        if r % 128 or st.blocksize != 64 or st.state2.blocksize != 256 or \
-                (cols is not None and c != cols) or _nf4._plan(w, device) is None:
-            return False
+        if r % 128 or (cols is not None and c != cols):
+            return None
+        plan = _nf4._plan_of(w, device, key)
+        if plan is None or plan[2:4] != (64, 256):
+            return None
         cols = c
-    return True
+        part_rows.append(r)
+        plans.append(plan)
+    return _Stack(part_rows, cols, plans)
 
 
 def _stack(weights, device):
@@ -60,9 +81,19 @@ def _stack(weights, device):
         return None
     kept = _nf4.Kept.of(weights[0], "_soupk_stack", keys)
     if kept is None:                # (a stack that the kernels do not read is kept as (None,))
-        kept = (_Stack(weights, device) if _readable(weights, device) else None,)
+        kept = (_make_stack(weights, device, keys),)
         _nf4.Kept.put(weights[0], "_soupk_stack", keys, kept)
     return kept[0]
+
+
+def _any_stack(weights, device):
+    """The _Stack of `weights` for a launch asked for outright: of weights that _make_stack does not
+    take too (the entry point checks their sizes)."""
+    st = _stack(weights, device)
+    if st is None:
+        shapes = [_nf4.weight_shape(w) for w in weights]
+        st = _Stack([r for r, _ in shapes], shapes[0][1], [_nf4._plan(w, device) for w in weights])
+    return st
 
 
 def _rows_fit(x, cols):
@@ -138,8 +169,7 @@ _cu_count.cache = {}
 def prefer_fused(x, weights):
     """True where the fused NF4 forward y = x W^T is the faster path (fused_fits)."""
     M, K = x.shape
-    st = _stack(weights, x.device)
-    N = st.rows if st is not None else sum(_nf4.weight_shape(w)[0] for w in weights)
+    N = sum([_nf4.weight_shape(w)[0] for w in weights])
     cus = _cu_count(x.device)
     return fused_fits(M, N, K, FWD_TILE, cus, forward_split_tiles(K, cus))
 
@@ -192,15 +222,6 @@ def gemm_tn(x, w16, bias=None):
     return y
 
 
-def _nf4_args(weights, device):
-    plans = [_nf4._plan(w, device) for w in weights]
-    rows = [_nf4.weight_shape(w)[0] for w in weights]
-    n = len(weights)
-    arrays = [(ctypes.c_void_p * n)(*[p[0][i] for p in plans]) for i in range(6)]
-    part_rows = (ctypes.c_int32 * n)(*rows)
-    return plans, rows, arrays, part_rows
-
-
 def grad_input_supported(dy, weights):
     """nf4_grad_input takes these: fp16 dy [M, N] with unit column stride and 16-byte aligned
     rows, 1-4 NF4 parts (blocksize 64, nested 256) of one column count, each a multiple of 128
@@ -217,7 +238,7 @@ def nf4_grad_input(dy, weights, splits=None):
     `splits` cuts the contraction over W's rows (soupk_gemm_nn_nf4_split; default: split_count
     for this device and the 128 x 64 tiles)."""
     M, N = dy.shape
-    st = _stack(weights, dy.device) or _Stack(weights, dy.device)
+    st = _any_stack(weights, dy.device)
     if st.rows != N:
         raise ValueError(f"dy has {N} columns, the weights {st.rows} rows")
     K = st.cols
@@ -296,7 +317,7 @@ def nf4_linear(x, weights, bias=None, splits=None):
     """x @ W^T (+ bias) for W the row stack of `weights`, dequantised in the GEMM; `splits`
     cuts the contraction (default: split_count for this device)."""
     M, K = x.shape
-    st = _stack(weights, x.device) or _Stack(weights, x.device)
+    st = _any_stack(weights, x.device)
     N = st.rows
     if bias is not None:
         _ext.require(bias, "bias", dtype=torch.float16, ndim=1, device=x.device)
