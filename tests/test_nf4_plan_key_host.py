@@ -75,3 +75,12 @@ def test_unsupported_state_is_checked_again():
     assert nf4_gemm._stack((w,), CPU) is None
     w.quant_state.quant_type = "nf4"
     assert nf4_gemm._stack((w,), CPU) is not None
+
+
+def test_keys_of_several_weights():
+    ws = [weight(i) for i in range(3)]
+    both = nf4._plan_keys(ws, CPU)
+    assert both[1] == b"".join(nf4._plan_key(w, CPU)[1] for w in ws)
+    ws[1].quant_state.state2.blocksize = 128
+    assert nf4._plan_keys(ws, CPU) != both
+    assert nf4._plan_keys([*ws, object()], CPU) is None and nf4._plan_keys([], CPU) is None

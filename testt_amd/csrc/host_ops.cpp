@@ -598,81 +598,97 @@ OP(gemm) {
   END_HANDLE_TH_ERRORS
 }
 
-// nf4_key(weight) -> bytes: everything a plan of an NF4 weight is made from and checked on -- for the
-// packed data and each state tensor its address, element count, type, device and whether it is
-// contiguous; the same of the offset, or its value when it is a number; the shape; both block sizes;
-// whether it is nested NF4.  None for an object without that state.
 struct Ref {
   PyObject* o;
   ~Ref() { Py_XDECREF(o); }
 };
 
-OP(nf4_key) {
-  HANDLE_TH_ERRORS
-  ARGS(1);
+constexpr int kKeyWords = 6 * 3 + 2 + 3;
+
+// Everything a plan of an NF4 weight is made from and checked on -- for the packed data and each
+// state tensor its address, element count, type, device and whether it is contiguous; the same of
+// the offset, or its value when it is a number; the shape; both block sizes; whether it is nested
+// NF4.  False (no Python error) for an object without that state.
+bool weight_key(PyObject* weight, uint64_t* key) {
   static PyObject* const names[] = {
       PyUnicode_InternFromString("quant_state"), PyUnicode_InternFromString("data"),
       PyUnicode_InternFromString("absmax"),      PyUnicode_InternFromString("code"),
       PyUnicode_InternFromString("state2"),      PyUnicode_InternFromString("offset"),
       PyUnicode_InternFromString("shape"),       PyUnicode_InternFromString("blocksize"),
       PyUnicode_InternFromString("quant_type"),  PyUnicode_InternFromString("nested")};
-  auto get = [](PyObject* o, int i) { return Ref{o ? PyObject_GetAttr(o, names[i]) : nullptr}; };
-  const Ref state = get(a[0], 0);
-  if (!state.o) {
+  auto none = [] {
     PyErr_Clear();
-    ELSE_PYTHON;
-  }
-  const Ref data = get(a[0], 1), absmax = get(state.o, 2), code = get(state.o, 3),
+    return false;
+  };
+  auto get = [](PyObject* o, int i) { return Ref{o ? PyObject_GetAttr(o, names[i]) : nullptr}; };
+  const Ref state = get(weight, 0);
+  if (!state.o) return none();
+  const Ref data = get(weight, 1), absmax = get(state.o, 2), code = get(state.o, 3),
             state2 = get(state.o, 4), offset = get(state.o, 5), shape = get(state.o, 6),
             block = get(state.o, 7), type = get(state.o, 8), nested = get(state.o, 9);
   const Ref code2 = get(state2.o, 3), absmax2 = get(state2.o, 2), block2 = get(state2.o, 7);
-  if (PyErr_Occurred()) {
-    PyErr_Clear();
-    ELSE_PYTHON;
-  }
-  uint64_t key[24];
-  int i = 0;
+  if (PyErr_Occurred()) return none();
   auto tensor = [&](PyObject* o) {
     const Tensor& t = THPVariable_Unpack(o);
     const at::Device d = t.device();
-    key[i++] = reinterpret_cast<uintptr_t>(t.data_ptr());
-    key[i++] = static_cast<uint64_t>(t.numel());
-    key[i++] = static_cast<uint64_t>(static_cast<uint8_t>(t.scalar_type())) |
-               static_cast<uint64_t>(t.is_contiguous()) << 8 |
-               static_cast<uint64_t>(static_cast<uint8_t>(d.type())) << 16 |
-               static_cast<uint64_t>(static_cast<uint8_t>(d.index())) << 24;
+    *key++ = reinterpret_cast<uintptr_t>(t.data_ptr());
+    *key++ = static_cast<uint64_t>(t.numel());
+    *key++ = static_cast<uint64_t>(static_cast<uint8_t>(t.scalar_type())) |
+             static_cast<uint64_t>(t.is_contiguous()) << 8 |
+             static_cast<uint64_t>(static_cast<uint8_t>(d.type())) << 16 |
+             static_cast<uint64_t>(static_cast<uint8_t>(d.index())) << 24;
   };
   for (PyObject* o : {data.o, absmax.o, code.o, code2.o, absmax2.o}) {
-    if (!THPVariable_Check(o)) ELSE_PYTHON;
+    if (!THPVariable_Check(o)) return false;
     tensor(o);
   }
   if (THPVariable_Check(offset.o)) {
     tensor(offset.o);
   } else {
     const double v = PyFloat_AsDouble(offset.o);
-    std::memcpy(&key[i++], &v, sizeof(v));
-    key[i++] = ~uint64_t{0};               // (no tensor)
-    key[i++] = ~uint64_t{0};
+    std::memcpy(key, &v, sizeof(v));
+    key[1] = key[2] = ~uint64_t{0};        // (no tensor)
+    key += 3;
   }
-  if (PySequence_Size(shape.o) != 2) {
-    PyErr_Clear();
-    ELSE_PYTHON;
-  }
+  if (PySequence_Size(shape.o) != 2) return none();
   for (Py_ssize_t d = 0; d < 2; ++d) {
     const Ref n{PySequence_GetItem(shape.o, d)};
-    key[i++] = n.o ? PyLong_AsUnsignedLongLongMask(n.o) : 0;
+    *key++ = n.o ? PyLong_AsUnsignedLongLongMask(n.o) : 0;
   }
-  key[i++] = PyLong_AsUnsignedLongLongMask(block.o);
-  key[i++] = PyLong_AsUnsignedLongLongMask(block2.o);
+  *key++ = PyLong_AsUnsignedLongLongMask(block.o);
+  *key++ = PyLong_AsUnsignedLongLongMask(block2.o);
   const int is_nested = PyObject_IsTrue(nested.o);
-  key[i++] = (is_nested == 1 ? 1u : 0u) |
-             (PyUnicode_Check(type.o) && !PyUnicode_CompareWithASCIIString(type.o, "nf4") ? 2u : 0u);
-  if (PyErr_Occurred()) {
-    PyErr_Clear();
-    ELSE_PYTHON;
+  *key = (is_nested == 1 ? 1u : 0u) |
+         (PyUnicode_Check(type.o) && !PyUnicode_CompareWithASCIIString(type.o, "nf4") ? 2u : 0u);
+  return PyErr_Occurred() ? none() : true;
+}
+
+// nf4_key(weight) -> bytes (weight_key), None for an object without that state.
+OP(nf4_key) {
+  HANDLE_TH_ERRORS
+  ARGS(1);
+  uint64_t key[kKeyWords];
+  if (!weight_key(a[0], key)) ELSE_PYTHON;
+  return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), sizeof(key));
+  END_HANDLE_TH_ERRORS
+}
+
+// nf4_keys(tuple of weights) -> bytes: their keys one after the other; None when there are none, or
+// one has none.
+OP(nf4_keys) {
+  HANDLE_TH_ERRORS
+  ARGS(1);
+  if (!PyTuple_Check(a[0])) return PyErr_Format(PyExc_TypeError, "a tuple of weights is expected");
+  const Py_ssize_t m = PyTuple_GET_SIZE(a[0]);
+  if (m == 0) ELSE_PYTHON;
+  const Ref out{PyBytes_FromStringAndSize(nullptr, m * kKeyWords * sizeof(uint64_t))};
+  if (!out.o) return nullptr;
+  for (Py_ssize_t i = 0; i < m; ++i) {
+    uint64_t key[kKeyWords];
+    if (!weight_key(PyTuple_GET_ITEM(a[0], i), key)) ELSE_PYTHON;
+    std::memcpy(PyBytes_AS_STRING(out.o) + i * sizeof(key), key, sizeof(key));
   }
-  static_assert(sizeof(key) >= (6 * 3 + 2 + 3) * sizeof(key[0]));
-  return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key), i * sizeof(key[0]));
+  return Py_NewRef(out.o);
   END_HANDLE_TH_ERRORS
 }
 
@@ -691,7 +707,7 @@ OP(set_status) {
 PyMethodDef methods[] = {
     SOUPK_ENTRIES(X) M(bind), M(set_status), M(rmsnorm_fwd), M(rmsnorm_bwd), M(rope_tokens),
     M(rope_fwd), M(rope_bwd), M(varlen_fwd), M(varlen_bwd), M(attn_fwd), M(attn_bwd),
-    M(swiglu_fwd), M(gemm), M(nf4_key), {nullptr, nullptr, 0, nullptr}};
+    M(swiglu_fwd), M(gemm), M(nf4_key), M(nf4_keys), {nullptr, nullptr, 0, nullptr}};
 #undef X
 #undef M
 

@@ -134,7 +134,10 @@ def nf4_resident(tokens, groups, device):
 
     if tokens <= 0 or not nf4.USE_FUSED_NF4_GEMM:
         return False
-    key = (tokens, device, tuple(nf4._plan_key(x, device) for g in groups for x in g))
+    keys = nf4._plan_keys([x for g in groups for x in g], device)
+    if keys is None:
+        return False                  # (not all of them NF4 weights)
+    key = (tokens, keys)
     first = groups[0][0]
     memo = getattr(first, "_soupk_resident", None)
     if memo is None:

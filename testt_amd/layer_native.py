@@ -129,7 +129,7 @@ def _nf4_layer(w, M, dev):
     from . import nf4
 
     weights = (w.q, w.k, w.v, w.o, w.gate, w.up, w.down)
-    key = (M, dev, tuple(nf4._plan_key(x, dev) for x in weights))
+    key = (M, nf4._plan_keys(weights, dev))
     memo = nf4.Kept.of(w.q, "_soupk_layer_nf4", None)
     if memo is None:
         memo = {}

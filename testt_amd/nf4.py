@@ -110,6 +110,13 @@ def _plan_key(weight, device):
     return None if key is None else (device, key)
 
 
+def _plan_keys(weights, device):
+    """The plan keys of several weights as one value, from one native call (None where one of them
+    has none)."""
+    keys = _ext.host().nf4_keys(tuple(weights))
+    return None if keys is None else (device, keys)
+
+
 class Kept:
     """What a call prepared for a weight, kept on it as an attribute: addresses, which mean nothing to
     a copy of the weight or to another process.  A copy or pickle of the weight holds an empty
@@ -144,11 +151,8 @@ def _plan(weight, device):
     weight whose state is replaced is checked again; the state tensors are kept with the plan,
     so that no other tensor can come to lie at an address of the key while it is in use."""
     key = _plan_key(weight, device)
-    return None if key is None else _plan_of(weight, device, key)
-
-
-def _plan_of(weight, device, key):
-    """_plan for a caller that has the weight's _plan_key."""
+    if key is None:
+        return None
     cached = Kept.of(weight, "_soupk_plan", key)
     if cached is not None:
         return cached

@@ -54,17 +54,16 @@ class _Stack:
 _args_lock = threading.Lock()
 
 
-def _make_stack(weights, device, keys):
-    """The _Stack of `weights`, whose plan keys are `keys`; None where the fused kernels do not read
-    them."""
+def _make_stack(weights, device):
+    """The _Stack of `weights`; None where the fused kernels do not read them."""
     if not 1 <= len(weights) <= MAX_PARTS:
         return None
     cols, part_rows, plans = None, [], []
-    for w, key in zip(weights, keys):
+    for w in weights:
         r, c = _nf4.weight_shape(w)
         if r % 128 or (cols is not None and c != cols):
             return None
-        plan = _nf4._plan_of(w, device, key)
+        plan = _nf4._plan(w, device)
         if plan is None or plan[2:4] != (64, 256):
             return None
         cols = c
@@ -75,13 +74,13 @@ def _make_stack(weights, device, keys):
 
 def _stack(weights, device):
     """The _Stack of `weights` on `device`, None where the fused kernels do not read them.  Kept on
-    the first weight and used while every weight's plan key (_nf4._plan_key) is unchanged."""
-    keys = [_nf4._plan_key(w, device) for w in weights]
-    if not keys or None in keys:
+    the first weight and used while every weight's plan key (_nf4._plan_keys) is unchanged."""
+    keys = _nf4._plan_keys(weights, device)
+    if keys is None:
         return None
     kept = _nf4.Kept.of(weights[0], "_soupk_stack", keys)
     if kept is None:                # (a stack that the kernels do not read is kept as (None,))
-        kept = (_make_stack(weights, device, keys),)
+        kept = (_make_stack(weights, device),)
         _nf4.Kept.put(weights[0], "_soupk_stack", keys, kept)
     return kept[0]
 
