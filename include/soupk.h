@@ -25,12 +25,13 @@
 extern "C" {
 #endif
 
-/* ABI version of this header; soupk_abi_version() returns the library's.  4 adds
+/* ABI version of this header; soupk_abi_version() returns the library's.  5 adds soupk_gemm_nn,
+   soupk_gemm_nn_workspace, soupk_head_plan, soupk_head_stats_grad_planned, soupk_head_finish and
+   soupk_head_dh to version 4's entry points, which had added
    soupk_lora_rope_fwd, soupk_gemm_nn_nf4, soupk_gemm_tn_nf4_split, soupk_gemm_nn_nf4_split,
    soupk_gemm_lt, soupk_gemm_lt_index, soupk_layer_fwd, soupk_layer_bwd (with the layer's
-   products on NF4 weights: SoupkLayerNf4) and soupk_init_device to version 3's entry
-   points. */
-#define SOUPK_ABI_VERSION 4
+   products on NF4 weights: SoupkLayerNf4) and soupk_init_device to version 3's. */
+#define SOUPK_ABI_VERSION 5
 
 /* Status of soupk_lora_bwd_params_noalloc for a problem beyond its static scratch (no launch). */
 #define SOUPK_STATUS_SCRATCH_LIMIT 20001

@@ -17,7 +17,7 @@ _lock = threading.Lock()
 _lib = None
 _host = None     # the CPython extension (csrc/host_ops.cpp), bound to the library's entry points
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 STATUS_SCRATCH_LIMIT = 20001          # SOUPK_STATUS_SCRATCH_LIMIT
 LORA_SCRATCH_FLOATS = 4 << 20         # SOUPK_LORA_SCRATCH_FLOATS
 DTYPE_F16 = 0
@@ -147,6 +147,10 @@ def _bind_host(handle):
         raise SoupkError(
             f"the host extension beside {_LIB_PATH} is missing or does not load ({exc}): build it "
             "with `python -m testt_amd.build_ext` (or __graft_entry__.build())") from exc
+    # (the entry points are called through the types that the extension was compiled with)
+    version = getattr(ext, "abi_version", lambda: None)()
+    if version != ABI_VERSION:
+        raise SoupkError(f"{ext.__file__}: ABI {version} != expected {ABI_VERSION}: rebuild")
     for name in SIGNATURES:
         fn = getattr(handle, name)
         if ext.bind(name, ctypes.cast(fn, ctypes.c_void_p).value):

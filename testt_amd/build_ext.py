@@ -61,7 +61,8 @@ def _compile(hipcc, src, build_dir, defines):
 
 def _build_host(hipcc, build_dir):
     """The CPython extension, against the installed torch's headers and libraries (host code
-    only; the kernels' library is bound to it at run time, not linked)."""
+    only; the kernels' library is bound to it at run time, not linked); returns the path of the
+    new file, for the caller to move to HOST_PATH."""
     import sysconfig
 
     import torch
@@ -85,7 +86,7 @@ def _build_host(hipcc, build_dir):
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"building {HOST_NAME} failed:\n{proc.stderr}")
-    os.replace(tmp, HOST_PATH)
+    return tmp
 
 
 def build(verbose=False, defines=(), out=None):
@@ -104,15 +105,18 @@ def build(verbose=False, defines=(), out=None):
     with ThreadPoolExecutor(jobs + 1) as pool:
         host = pool.submit(_build_host, hipcc, build_dir) if out is None else None
         objs = list(pool.map(lambda s: _compile(hipcc, s, build_dir, defines), srcs))
-        if host is not None:
-            host.result()
+        new_host = host.result() if host is not None else None
     tmp = lib_path + ".tmp"
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp,
            "-lhipblaslt"]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link of {LIB_NAME} failed:\n{proc.stderr}")
+    # (both only once both are built: the extension calls the library through its own copy of the
+    # header's types)
     os.replace(tmp, lib_path)
+    if new_host is not None:
+        os.replace(new_host, HOST_PATH)
     if verbose:
         print(f"built {lib_path} from {len(srcs)} sources", flush=True)
     return lib_path

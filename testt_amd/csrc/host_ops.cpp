@@ -692,6 +692,12 @@ OP(nf4_keys) {
   END_HANDLE_TH_ERRORS
 }
 
+// abi_version() -> the version of soupk.h that this file's function types were compiled from
+OP(abi_version) {
+  ARGS(0);
+  return PyLong_FromLong(SOUPK_ABI_VERSION);
+}
+
 // set_status(SoupkError, address of soupk_status_string)
 OP(set_status) {
   ARGS(2);
@@ -707,7 +713,7 @@ OP(set_status) {
 PyMethodDef methods[] = {
     SOUPK_ENTRIES(X) M(bind), M(set_status), M(rmsnorm_fwd), M(rmsnorm_bwd), M(rope_tokens),
     M(rope_fwd), M(rope_bwd), M(varlen_fwd), M(varlen_bwd), M(attn_fwd), M(attn_bwd),
-    M(swiglu_fwd), M(gemm), M(nf4_key), M(nf4_keys), {nullptr, nullptr, 0, nullptr}};
+    M(swiglu_fwd), M(gemm), M(nf4_key), M(nf4_keys), M(abi_version), {nullptr, nullptr, 0, nullptr}};
 #undef X
 #undef M
 
