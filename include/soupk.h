@@ -26,8 +26,8 @@ extern "C" {
 #endif
 
 /* ABI version of this header; soupk_abi_version() returns the library's.  5 adds soupk_gemm_nn,
-   soupk_gemm_nn_workspace, soupk_head_plan, soupk_head_stats_grad_planned, soupk_head_finish and
-   soupk_head_dh to version 4's entry points, which had added
+   soupk_gemm_nn_workspace, soupk_head_plan, soupk_head_stats_grad_planned, soupk_head_finish,
+   soupk_head_dh and soupk_attention_wide to version 4's entry points, which had added
    soupk_lora_rope_fwd, soupk_gemm_nn_nf4, soupk_gemm_tn_nf4_split, soupk_gemm_nn_nf4_split,
    soupk_gemm_lt, soupk_gemm_lt_index, soupk_layer_fwd, soupk_layer_bwd (with the layer's
    products on NF4 weights: SoupkLayerNf4) and soupk_init_device to version 3's. */
@@ -511,6 +511,12 @@ int soupk_gemm_lt(int32_t trans_a, int32_t trans_b, int64_t m, int64_t n, int64_
                   int64_t ldb, int64_t stride_b, void* D, int64_t ldd, int64_t stride_d,
                   int32_t d_f32, int32_t batch, int32_t accumulate, const uint16_t* bias,
                   int32_t algo_index, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* Whether the attention entry points take their 128-query kernels (*wide = 1) or their 64-query
+   kernels (0) on a device of `cus` compute units; the results are the same bits.  len: T of the
+   padded layout, all M tokens of the varlen one.  Host only, no launch. */
+int soupk_attention_wide(int32_t varlen, int32_t backward, int32_t B, int64_t len, int32_t NH,
+                         int32_t cus, int32_t* wide);
 
 /* The hipBLASLt solution index a soupk_gemm_lt problem runs with, -1 before its first call
    (the same arguments, without the pointers and the stream; has_bias for the bias). */

@@ -53,6 +53,7 @@ SIGNATURES = {
     "soupk_bench_copy": [_p, _p, _i64, _p],
     "soupk_bench_empty": [_i32, _p],
     "soupk_bench_hold": [ctypes.c_double, _p],
+    "soupk_attention_wide": [_i32, _i32, _i32, _i64, _i32, _i32, _p],
     "soupk_attention_fwd": [_p, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _f32, _p],
     "soupk_attention_bwd": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i32, _i32, _i32, _i32,
                             _i32, _f32, _p],

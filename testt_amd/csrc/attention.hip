@@ -978,7 +978,7 @@ template <int U>
 constexpr int kBwdLdsBytes = U * (2 * kBK * kRStride * 2 + 2 * kBQ * 4);
 
 // Grid z = (U + 1) * (64 U-query slots): of U + 1 z, one dQ of 64 U queries and U dK/dV of 64 keys, the
-// heaviest causal blocks of both kinds first.  U = 2 by the 128-query forward's rule (wide_forward).
+// heaviest causal blocks of both kinds first.  U = 2 by wide_padded and wide_varlen.
 // Against 64-query dQ workgroups on single LDS tiles with two barriers a block (delta and reduce
 // launches included, 12 heads, us): 2 x 4096 tokens 537 -> 452, 1 x 8000 907 -> 814, rows of 4096 to
 // 1024 477 -> 406, 4 x 1024 100 -> 94, 16 x 256 82 -> 72; rows of 512 to 128 tokens keep
@@ -1124,14 +1124,48 @@ int check_varlen(int32_t B, int64_t M, int32_t NH, int32_t NKV, int32_t D, float
   return kOk;
 }
 
-// Whether the 128-query forward takes `units` (sequence, head) pairs of `len` rows on average:
-// where its workgroups are at least 5/4 of the CUs.  Below, the 64-query kernel's shorter chains
-// fill the chip better.  Measured (us, 64 / 128 queries per workgroup, 12 heads): 2 x 4096 rows 222 /
-// 141, 1 x 4096 (384 workgroups) 124 / 116, 16 x 256 (384) 29.9 / 17.8, 4 x 1024 (384) 40.6 / 34.0,
-// 2 rows of 2500 and 800 (312) 76 / 75, 1 x 3000 (288) 75 / 82, 2 x 1365 (264) 36 / 42, 4 x 512 (192)
-// 15.4 / 20.5.
-bool wide_forward(int64_t units, int64_t len) {
-  return units * ((len + kWideBQ - 1) / kWideBQ) * 4 >= int64_t{5} * device_cu_count();
+// Which kernels take a launch: the 128-query ones (`wide`) or the 64-query ones, whose shorter chains
+// fill the chip better where there are few workgroups.  Both give the same bits.  All times: us on
+// MI355X (256 CUs), 64- / 128-query kernels, best of graph replays, 12 heads where none are named.
+//
+// The 128-query workgroups must come to 5/4 of the CUs at least, a varlen row counted at the average
+// length (the lengths are on the device).  Forward: 2 x 4096 rows 222 / 141, 1 x 4096 (384
+// workgroups) 124 / 116, 16 x 256 (384) 29.9 / 17.8, 4 x 1024 (384) 40.6 / 34.0, 1 x 3000 (288) 75 / 82,
+// 2 x 1365 (264) 36 / 42, 4 x 512 (192) 15.4 / 20.5.  Then, per layout and direction:
+struct WideRule {
+  int64_t units, cus;      // (row, head) pairs
+  bool fills(int64_t len) const { return units * ((len + kWideBQ - 1) / kWideBQ) * 4 >= 5 * cus; }
+};
+
+// Padded rows of T positions.  Forward: five sixths of the workgroups' 64-query halves must hold
+// queries, or the workgroups come to 3.5 CUs (rows of 160: 14 rows 14.3 / 15.8, 22 rows 22.7 / 24.4, 40
+// rows 35.4 / 31.0; of 192: 15.0 / 16.2, 23.7 / 25.6, 37.1 / 32.9; of 64: 43 rows 15.4 / 16.4, 80 rows
+// 22.9 / 21.5; of 96, 28 rows: 16.6 / 14.9; of 256, 14 rows: 20.9 / 19.4; of 320: 28.5 / 28.6).
+// Backward: more than five 64-key blocks (64 rows of 64: 50.6 / 54.6, 128 of 32: 54.4 / 65.1, 32 of 100:
+// 46.3 / 49.6, 14 of 192: 42.7 / 45.2, 40 of 256: 131 / 135, 10 of 320: 53.6 / 56.5; 10 of 384: 64.4 /
+// 62.5, 7 of 512: 68.0 / 64.5, 4 x 1024: 106 / 89).
+bool wide_padded(bool backward, int64_t B, int64_t T, int64_t NH, int64_t cus) {
+  const WideRule r{B * NH, cus};
+  if (!r.fills(T)) return false;
+  const int64_t halves = (T + kBQ - 1) / kBQ, wgs = (T + kWideBQ - 1) / kWideBQ;
+  return backward ? halves > 5 : halves * 6 >= wgs * 10 || r.units * wgs * 2 >= 7 * cus;
+}
+
+// Varlen rows, M tokens in all.  A grid has block slots for a row of all M tokens in every row, and
+// a slot past a row's end costs about 1 ns: from 16 CUs of 64-query slots on, half as many of them
+// decide (27 rows of 64: 16.8 / 10.6, 64 rows of 64: 60.9 / 28.1).  Below that the tokens alone must
+// fill the CUs 7/6 times, backward 17/16: with fewer, the average counts workgroups that a ragged
+// batch does not have (forward, rows of 1696, 848 and 565 tokens, 291 workgroups of tokens: 45.9 / 51.5;
+// 1504, 752, 501, 376, 293: 40.2 / 45.3; 14 heads, 8 rows of 1120 to 140, 229: 28.6 / 35.6; 28 heads,
+// rows of 512 to 128, 233: 19.0 / 20.9, backward 46.8 / 48.5; 40 heads, rows of 448 to 149, backward, 256:
+// 48.7 / 51.8).  A long row beside short ones can still come out behind (rows of 3104, 388 and 388: 88
+// / 96), even rows and most ragged ones gain (4 x 1024 40.6 / 34.0, rows of 2592 and 1296: 80.6 / 71.9).
+bool wide_varlen(bool backward, int64_t B, int64_t M, int64_t NH, int64_t cus) {
+  const WideRule r{B * NH, cus};
+  if (B <= 0 || !r.fills(M / B)) return false;
+  const int64_t slots = r.units * ((M + kBQ - 1) / kBQ);
+  return slots >= 16 * cus || (backward ? 16 * NH * M >= 17 * cus * kWideBQ
+                                        : 6 * NH * M >= 7 * cus * kWideBQ);
 }
 
 // The dQ and dK/dV launch over block slots for sequences of up to `len` rows.
@@ -1160,6 +1194,15 @@ AttnParams base_params(int32_t NH, int32_t NKV, float scale) {
 
 using namespace soupk;
 
+extern "C" __attribute__((visibility("default"))) int soupk_attention_wide(
+    int32_t varlen, int32_t backward, int32_t B, int64_t len, int32_t NH, int32_t cus,
+    int32_t* wide) {
+  if (B < 0 || len < 0 || NH <= 0 || cus <= 0 || !wide) return kInvalid;
+  *wide = varlen ? wide_varlen(backward != 0, B, len, NH, cus)
+                 : wide_padded(backward != 0, B, len, NH, cus);
+  return kOk;
+}
+
 extern "C" __attribute__((visibility("default"))) int soupk_attention_fwd(
     const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint8_t* key_valid,
     uint16_t* out, float* lse, int32_t B, int32_t T, int32_t NH, int32_t NKV, int32_t D,
@@ -1179,7 +1222,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_fwd(
   p.out = out;
   p.lse = lse;
   p.T = T;
-  if (wide_forward(static_cast<int64_t>(B) * NH, T))
+  if (wide_padded(false, B, T, NH, device_cu_count()))
     return launch_kernel(attn_fwd_wide_kernel<false>,
                          dim3(static_cast<unsigned>(NH), static_cast<unsigned>(B),
                               static_cast<unsigned>((T + kWideBQ - 1) / kWideBQ)),
@@ -1229,7 +1272,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_bwd(
   int rc = launch_kernel(attn_bwd_delta_kernel, grid, dim3(kAttnThreads), st, out, dout,
                          p.delta, T, NH);
   if (rc != kOk) return rc;
-  rc = launch_bwd<false>(p, B, NH, T, wide_forward(static_cast<int64_t>(B) * NH, T), st);
+  rc = launch_bwd<false>(p, B, NH, T, wide_padded(true, B, T, NH, device_cu_count()), st);
   if (rc != kOk) return rc;
   const int64_t n4 = static_cast<int64_t>(B) * NKV * per_head / 4;
   return launch_kernel(attn_bwd_reduce_kernel, dim3(static_cast<unsigned>((n4 + 255) / 256)),
@@ -1252,7 +1295,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_varlen_fwd
   p.M = M;
   p.W = static_cast<int64_t>(NH + 2 * NKV) * kD;
   const int slots = static_cast<int>((M + kBQ - 1) / kBQ);
-  if (wide_forward(static_cast<int64_t>(B) * NH, M / B))   // (slots for a sequence of all M tokens)
+  if (wide_varlen(false, B, M, NH, device_cu_count()))   // (slots for a sequence of all M tokens)
     return launch_kernel(attn_fwd_wide_kernel<true>,
                          dim3(static_cast<unsigned>(NH), static_cast<unsigned>(B),
                               static_cast<unsigned>((M + kWideBQ - 1) / kWideBQ)),
@@ -1314,7 +1357,7 @@ extern "C" __attribute__((visibility("default"))) int soupk_attention_varlen_bwd
   if (rc != kOk) return rc;
   if (B > 0) {
     // (slots for a sequence of all M tokens)
-    rc = launch_bwd<true>(p, B, NH, M, wide_forward(static_cast<int64_t>(B) * NH, M / B), st);
+    rc = launch_bwd<true>(p, B, NH, M, wide_varlen(true, B, M, NH, device_cu_count()), st);
     if (rc != kOk) return rc;
   }
   const int64_t items = M * NKV * 16;
