@@ -1,13 +1,15 @@
 """CPU regression test: the varlen attention kernels' index arithmetic stays in bounds.
 
-testt_amd/csrc/attention.hip launches the varlen forward on a (heads, sequences, ceil(M/64))
-grid, or of 128-query blocks on (heads, sequences, ceil(M/128)), the backward on (heads,
-sequences, 3 ceil(M/128)) (of three z, two dK/dV of a key block, one dQ of 128 queries), the delta kernel on (heads, 1, ceil(M/64)) and the reduce on M*NKV*16
-items.  Workgroups past a sequence's blocks exit; rows are clamped to the sequence's last row
+testt_amd/csrc/attention.hip launches the varlen forward and backward in two forms, of 64 U queries
+per workgroup, U = 1 or 2 (soupk_attention_wide chooses): the forward on a (heads, sequences,
+ceil(M / 64U)) grid, the backward on (heads, sequences, (U + 1) ceil(M / 64U)) (of U + 1 z, U dK/dV
+of a key block and one dQ of 64 U queries); the delta kernel on (heads, 1, ceil(M/64)) and the
+reduce on M*NKV*16 items.  Both forms are replayed for every shape.  Workgroups past a sequence's blocks exit; rows are clamped to the sequence's last row
 before every load; sequence bounds come from device memory (cu_seqlens) and a bound outside
 [0, M] empties the sequence.  This test replays that arithmetic with numpy for every workgroup
-and lane and checks each global index against its buffer, for ragged batches, an empty
-sequence, T = 77, single tokens and malformed bounds.  No GPU is needed.
+and lane and checks each global index against its buffer, and that each query and key block is
+taken exactly once, for ragged batches, an empty sequence, T = 77, single tokens and malformed
+bounds.  No GPU is needed.
 """
 
 import numpy as np
@@ -48,6 +50,60 @@ def _check_tile(r0, length, base, W, col0, limit):
             row = np.minimum(r0 + r, length - 1)
             idx = (base + row) * W + col0 + 8 * dc + 7
             assert idx.min() >= 0 and idx.max() < limit, (r0, length, idx.max(), limit)
+
+
+def _replay_backward(U, h, g, b, length, base, M, W, HD, D_rope, limits, NH, NKV):
+    """attn_bwd_kernel<true, U> of one (head, sequence)."""
+    qkv_n, out_n, lse_n, part_n = limits
+    w, ql, gr = _lanes()
+    nb, nw = -(-length // BK), -(-length // (64 * U))
+    key_blocks, query_blocks = [], []
+    for z in range((U + 1) * -(-M // (64 * U))):
+        zq, zr = z // (U + 1), z % (U + 1)
+        if zr < U:
+            kb = U * zq + zr
+            if kb >= nb:
+                continue
+            key_blocks.append(kb)
+            key = kb * BK + 16 * w + ql
+            kc = np.minimum(key, length - 1)
+            assert ((base + kc) * W + (NH + NKV + g) * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
+            for qb in range(kb, nb + 1):                 # + the clamped prefetch
+                _check_tile(qb * BQ, length, base, W, h * D, qkv_n)      # Q
+                _check_tile(qb * BQ, length, base, HD, h * D, out_n)     # dO
+                t = np.minimum(qb * BQ + (np.arange(256) & 63), length - 1)
+                assert (h * M + base + t).max() < lse_n               # lse, D
+            st = key < length
+            if st.any():
+                assert ((h * M + base + key[st]) * D + 16 * 7 + 4 * gr[st] + 3).max() < part_n
+        else:
+            qb = nw - 1 - zq
+            if qb < 0:
+                continue
+            query_blocks.append(qb)
+            n_kb = min(U * (qb + 1), nb)
+            for u in range(U):
+                q_abs = qb * 64 * U + 16 * U * w + 16 * u + ql
+                qc = np.minimum(q_abs, length - 1)
+                assert ((base + qc) * W + h * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
+                assert ((base + qc) * HD + h * D + 32 * 3 + 8 * gr + 7).max() < out_n
+                assert (h * M + base + qc).max() < lse_n
+                st = q_abs < length
+                # a stored query's own key block is among those staged, and is the wavefront's last
+                assert (q_abs[st] // BK < n_kb).all()
+                assert (q_abs[st] // BK == ((qb * 64 * U + 16 * U * w) // BK)[st]).all()
+                if st.any():
+                    tok = base + q_abs[st]
+                    assert tok.max() < M
+                    # dQ row, first and second half (RoPE's transposed rotation)
+                    assert (tok * W + h * D + 16 * 3 + 4 * gr[st] + 64 + 3).max() < qkv_n
+                    if D_rope is not None:
+                        # table row t < T_rope, dims d .. d+3 and d+64 .. d+67, d <= 60
+                        assert 60 + 64 + 3 < D
+            for kb in range(n_kb + 1):
+                _check_tile(kb * BK, length, base, W, (NH + g) * D, qkv_n)
+                _check_tile(kb * BK, length, base, W, (NH + NKV + g) * D, qkv_n)
+    assert sorted(key_blocks) == list(range(nb)) and sorted(query_blocks) == list(range(nw))
 
 
 def replay(cu, M, NH, NKV, T_rope=None):
@@ -99,49 +155,11 @@ def replay(cu, M, NH, NKV, T_rope=None):
                 for kb in range(n_kb + 1):
                     _check_tile(kb * BK, length, base, W, (NH + g) * D, qkv_n)
                     _check_tile(kb * BK, length, base, W, (NH + NKV + g) * D, qkv_n)
-            # backward, z = 3 zq + zr: zr < 2 -> dK/dV of key block 2 zq + zr, zr = 2 -> dQ of
-            # 128-query block nw - 1 - zq
-            for z in range(3 * -(-M // 128)):
-                zq, zr = z // 3, z % 3
-                if zr < 2:
-                    kb = 2 * zq + zr
-                    if kb >= nb:
-                        continue
-                    key = kb * BK + 16 * w + ql
-                    kc = np.minimum(key, length - 1)
-                    assert ((base + kc) * W + (NH + NKV + g) * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
-                    for qb in range(kb, nb + 1):                 # + the clamped prefetch
-                        _check_tile(qb * BQ, length, base, W, h * D, qkv_n)      # Q
-                        _check_tile(qb * BQ, length, base, HD, h * D, out_n)     # dO
-                        t = np.minimum(qb * BQ + (np.arange(256) & 63), length - 1)
-                        assert (h * M + base + t).max() < lse_n               # lse, D
-                    st = key < length
-                    if st.any():
-                        assert ((h * M + base + key[st]) * D + 16 * 7 + 4 * gr[st] + 3).max() < part_n
-                else:
-                    qb = nw - 1 - zq
-                    if qb < 0:
-                        continue
-                    n_kb = min(2 * qb + 2, -(-length // BK))
-                    for u in range(2):
-                        q_abs = qb * 128 + 32 * w + 16 * u + ql
-                        qc = np.minimum(q_abs, length - 1)
-                        assert ((base + qc) * W + h * D + 32 * 3 + 8 * gr + 7).max() < qkv_n
-                        assert ((base + qc) * HD + h * D + 32 * 3 + 8 * gr + 7).max() < out_n
-                        assert (h * M + base + qc).max() < lse_n
-                        st = q_abs < length
-                        assert (q_abs[st] // BK < n_kb).all()
-                        if st.any():
-                            tok = base + q_abs[st]
-                            assert tok.max() < M
-                            # dQ row, first and second half (RoPE's transposed rotation)
-                            assert (tok * W + h * D + 16 * 3 + 4 * gr[st] + 64 + 3).max() < qkv_n
-                            if T_rope is not None:
-                                # table row t < T_rope, dims d .. d+3 and d+64 .. d+67, d <= 60
-                                assert 60 + 64 + 3 < D
-                    for kb in range(n_kb + 1):
-                        _check_tile(kb * BK, length, base, W, (NH + g) * D, qkv_n)
-                        _check_tile(kb * BK, length, base, W, (NH + NKV + g) * D, qkv_n)
+            # backward, z = (U + 1) zq + zr: zr < U -> dK/dV of key block U zq + zr, zr = U -> dQ
+            # of query block nw - 1 - zq, 64 U queries
+            for U in (1, 2):
+                _replay_backward(U, h, g, b, length, base, M, W, HD, D_rope=T_rope,
+                                 limits=(qkv_n, out_n, lse_n, part_n), NH=NH, NKV=NKV)
     # delta: the padded kernel over one row of M positions (b = 0, T = M)
     for h in range(NH):
         for qb in range(slots):
@@ -170,7 +188,25 @@ CASES = [
     ((77,), 12, 2),
     ((1, 1, 1), 4, 4),
     ((130, 64, 63, 65), 8, 2),
+    ((130, 64, 63, 65, 1) * 4, 16, 2),      # (the rule sends this one to U = 2)
 ]
+
+
+def test_cases_reach_both_forms():
+    """The rule (256 compute units) takes U = 1 for some of the cases and U = 2 for some, forward and
+    backward."""
+    import ctypes
+
+    from testt_amd import _ext
+
+    for backward in (0, 1):
+        taken = set()
+        for lengths, NH, _ in CASES:
+            out = ctypes.c_int32(-1)
+            _ext.call("soupk_attention_wide", 1, backward, len(lengths), sum(lengths), NH, 256,
+                      ctypes.addressof(out))
+            taken.add(out.value)
+        assert taken == {0, 1}, backward
 
 
 @pytest.mark.parametrize("lengths,NH,NKV", CASES)
