@@ -148,6 +148,20 @@ def gemm_nn_fits(a, b, out):
             and _aligned(a, b, out))
 
 
+def library_ahead(rows, cols, cus):
+    """True where hipBLASLt measured ahead of gemm_nn for a [rows, cols] output over a vocabulary:
+    where its 256 x 256 tiles are 3, 4, 6 or 8 eighths of the `cus` compute units, so that tiles of
+    24, 32, 48 or 64 Ki values cover the output in one full round.  MI355X, us, gemm_nn / hipBLASLt,
+    contraction 128256: 2048 x 3072 1766 / 1445, 1536 x 4096 1532 / 1407, 2048 x 4096 2074 / 1761, 1024
+    x 6144 1783 / 1457, 2048 x 6144 3466 / 2822, 768 x 8192 1562 / 1441, 1024 x 8192 2081 / 1762,
+    1536 x 8192 2960 / 2737, 2048 x 8192 4029 / 3409; at 32000 and 151936 the same shapes, by as
+    much.  Elsewhere from 256 to 2048 rows and 896 to 8192 columns gemm_nn is ahead or level (2048
+    x 1536 821 / 1083, 2048 x 2560 1356 / 1665, 2048 x 5120 2837 / 2927, 1024 x 4096 1063 / 1493;
+    behind only at 1280 x 8192, 2638 / 2410)."""
+    tiles = -(-rows // 256) * -(-cols // 256)
+    return cols % 256 == 0 and 8 * tiles in (3 * cus, 4 * cus, 6 * cus, 8 * cus)
+
+
 def gemm_nn(a, b, out, rows=None):
     """out [M, N] = a [M, K] @ b [K, N] through soupk_gemm_nn (this package's split-K kernel: a few
     hundred rows contracted over a very long K), each row-major with unit column stride.  `rows`:

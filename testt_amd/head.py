@@ -33,6 +33,7 @@ import torch
 
 from . import _ext
 from . import blas as _blas
+from .nf4_gemm import _cu_count
 
 CHUNK_ROWS = 2048
 # Vocabulary tile of the reference's Triton loop (solution/head.py:30); the HIP kernel streams
@@ -113,9 +114,10 @@ def _hidden_grad(g, weight, out):
     """out [n, H] = g [n, V] @ weight [V, H]: the split-K kernel for this shape (blas.gemm_nn: the
     output is a few tiles and the contraction the whole vocabulary, which leaves a library GEMM
     on part of the chip; 18 rows 326 -> 92 us, 420 rows 580 -> 249 us, 1536 rows 935 -> 686 us on
-    MI355X at 151936 x 1536, never slower from 1 to 2048 rows), hipBLASLt for operands it does
-    not take."""
-    if _blas.gemm_nn_fits(g, weight, out):
+    MI355X at 151936 x 1536), hipBLASLt where its tiles fill the chip (blas.library_ahead) and for
+    operands that kernel does not take."""
+    if _blas.gemm_nn_fits(g, weight, out) and \
+            not _blas.library_ahead(out.shape[0], out.shape[1], _cu_count(g.device)):
         _blas.gemm_nn(g, weight, out)
     else:
         torch.matmul(g, weight, out=out)
@@ -169,10 +171,20 @@ def _denominator_args(denominator, device):
     return None
 
 
+# From this many multiply-adds of the hidden gradient on, what hipBLASLt gains where it is ahead
+# (15 - 20% of that product) is more than the general form's row plan and its wait cost (0.2 - 0.3
+# ms).  Forward + backward on MI355X, every row labelled, without the wait / general: 128256 x 3072 at
+# 2048 rows (0.81e12) 3512 / 3130 us; 128256 x 4096 at 2048 rows (1.08e12) 3984 / 3829, at 4096 rows
+# 7995 / 7487; 32000 x 8192 at 2048 rows (0.54e12) 1890 / 1877, at 4096 rows (1.07e12) 3718 / 3594;
+# 32000 x 4096 at 4096 rows (0.54e12) 2015 / 2057.
+_LIBRARY_MIN_MACS = 7 * 10 ** 11
+
+
 def _device_plan(hidden, weight, denominator):
     """The arguments of the forward without a host synchronisation, or None where the general
     form runs: fp16 rows and head on one device, a vocabulary whose rows are whole 16-byte chunks
-    (the gradient rows keep the logits rows' alignment) and operands gemm_nn takes.  An autocast
+    (the gradient rows keep the logits rows' alignment), operands gemm_nn takes, and sizes at which
+    knowing the labelled rows, to give their product to hipBLASLt, does not pay.  An autocast
     to another type stays with the general form, which refuses the logits that it makes."""
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
         return None
@@ -183,6 +195,9 @@ def _device_plan(hidden, weight, denominator):
             not weight.is_contiguous() or weight.dim() != 2 or weight.shape[1] != width or \
             vocab % 8 or width % 8 or weight.data_ptr() % 16 or vocab * width >= 1 << 30 or \
             min(rows, CHUNK_ROWS) * vocab >= 1 << 30:
+        return None
+    if rows * vocab * width >= _LIBRARY_MIN_MACS and \
+            _blas.library_ahead(min(rows, CHUNK_ROWS), width, _cu_count(hidden.device)):
         return None
     return _denominator_args(denominator, hidden.device)
 
