@@ -2,6 +2,7 @@
 sequence bounds of the varlen attention (testt_amd/attention.py: cu_seqlens_of), checked against
 direct constructions on small cases (no kernel runs)."""
 
+import pytest
 import torch
 
 from testt_amd import attention, head
@@ -76,3 +77,17 @@ def test_cu_seqlens_of_sorted_positions():
     mask = torch.tensor([[0, 0, 1, 1], [0, 1, 1, 1]])
     pos = mask.reshape(-1).nonzero().squeeze(1)
     assert attention.cu_seqlens_of(pos, 2, 4).tolist() == [0, 2, 5]
+
+
+def test_no_rows_take_targets_of_any_shape():
+    weight = torch.zeros(16, 8, dtype=torch.float16)
+    for shape in ((0,), (0, 1), (1, 0)):
+        hidden = torch.zeros(0, 8, dtype=torch.float16, requires_grad=True)
+        loss, entropy, token_loss, correct = head.FusedHeadLoss.apply(
+            hidden, weight, torch.zeros(shape, dtype=torch.int64), 1)
+        loss.backward()
+        assert float(loss) == 0 and entropy.numel() == token_loss.numel() == correct.numel() == 0
+        assert hidden.grad.shape == (0, 8)
+    with pytest.raises(ValueError, match="1 dim"):
+        head.FusedHeadLoss.apply(torch.zeros(2, 8, dtype=torch.float16), weight,
+                                 torch.zeros(1, 2, dtype=torch.int64), 1)

@@ -272,7 +272,7 @@ class FusedHeadLoss(torch.autograd.Function):
         vocab = weight.shape[0]
         dev = hidden.device
         targets = targets.to(torch.int64).contiguous()
-        if targets.dim() != 1:
+        if rows and targets.dim() != 1:      # (no rows: any targets, as there are none to read)
             raise ValueError(f"targets must have 1 dim, got shape {tuple(targets.shape)}")
         den = _device_plan(hidden, weight, denominator)
         if den is not None and targets.device == dev and targets.numel() == rows:
