@@ -10,7 +10,7 @@
 // All three are bound by launch latency at the sizes of a training step (2048 rows: 16 KB of
 // labels, 12 MB of gradient); what they replace is about 30 torch launches of 2 - 5 us each, one
 // device-to-host copy and its wait (head loss forward + backward at 24 rows 406 -> 217 us, at 700
-// rows 924 -> 689 us on MI355X).
+// rows 924 -> 698 us on MI355X).
 
 #include "soupk_common.hpp"
 

@@ -5,8 +5,9 @@
 // Reason: a training program's small calls are bound by the host.  Through ctypes an entry point of
 // 16 arguments costs about 2 us more than its launch, and the checks and torch.empty calls around it
 // 10 - 20 us of Python.  Eager forward + backward on MI355X, before and after (us): add + RMSNorm of 300
-// rows 49 / 36, q|k|v projection of 16 rows 71 / 51, RoPE + attention of rows of 512 to 128 tokens 67
-// / 49, the padded form 122 / 95.
+// rows 49 / 36, q|k|v projection of 16 rows 71 / 51 (its first pass on new weights, whose launch
+// arguments are made then, 189 / 181), RoPE + attention of rows of 512 to 128 tokens 67 / 49, the
+// padded form 122 / 95.  A GEMM takes its native call only while no tuned table is loaded.
 //
 // An operator here takes only the common case -- plain tensors of the expected types, contiguous, on
 // one device, with matching shapes -- and returns None for anything else; the Python caller then

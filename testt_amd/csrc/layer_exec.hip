@@ -223,9 +223,10 @@ extern "C" __attribute__((visibility("default"))) int soupk_layer_bwd(
                                   a->lora_ws_floats, a->d_aq, a->d_av, a->d_bq, a->d_bv, M, H, NQ,
                                   NV, dm->r, stream));
   // dy += dqkv @ W_qkv (NF4: added by the kernel that sums the contraction's parts; uncut, the
-  // product into g_o's buffer, dead since the o input gradient, then added).  With few tokens the
-  // layer is bound by the host's launches; one fewer took 63 tokens, forward + backward, from 201
-  // to 197 us on MI355X, identical bits.
+  // product into g_o's buffer, dead since the o input gradient, then added).  One launch fewer: the
+  // captured layer, forward + backward on MI355X, 16 tokens 168.7 -> 166.9 us, 63 tokens 178.6 ->
+  // 177.6, 128 tokens 214.6 -> 211.9; issued eagerly it is bound by the host's launches at 63 tokens,
+  // and the 195 to 200 us there do not tell the two apart.  Identical bits.
   if (n4 && n4->split_bwd[0] > 1) {
     const SoupkNf4Group& g = n4->qkv;
     SOUPK_TRY(soupk::gemm_nn_nf4_split_add(

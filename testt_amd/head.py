@@ -7,24 +7,28 @@ Design.  The rows (real tokens) are taken in their own order, CHUNK_ROWS at a ti
    (running max, sum of exp, sum of exp * z and the first argmax, which give logsumexp,
    entropy = lse - sum(p z), the token loss lse - z[label] and whether the argmax is the label),
    stored straight at the row's place in the outputs, and for a labelled row the gradient
-   (softmax - onehot) * scale in fp16, written to the row's slot in a buffer that holds only the
-   chunk's labelled rows (the slot comes from a row map, -1 for an ignored row);
-3. testt_amd/csrc/gemm_nn.hip: dh = that buffer @ W, the contraction over the vocabulary cut into
-   parts that fill the chip, appended to one packed [labelled, H] gradient.
+   (softmax - onehot) * scale in fp16, written to the row's slot in a [chunk, V] buffer whose
+   leading rows hold the chunk's labelled rows (the slot comes from a row map, -1 for an ignored
+   row);
+3. testt_amd/csrc/gemm_nn.hip: dh = those rows @ W, the contraction over the vocabulary cut into
+   parts that fill the chip (their fp32 partial sums: up to 67 MB), into the leading rows of the
+   chunk's part of an [M, H] gradient.
 The row map, the per-chunk labelled counts and the gradient's scale stay on the device
 (testt_amd/csrc/head_plan.hip; the dh kernel reads the count it covers), so the whole head is
-enqueued without waiting for the GPU; a vocabulary or denominator this form does not take keeps
-a row plan read back to the host (_RowPlan).  No row is ever permuted: the hidden states are read
+enqueued without waiting for the GPU, and the buffers have a row for every row, labelled or not.  A
+vocabulary or denominator this form does not take, and sizes at which the library's product of
+the labelled rows alone is faster (_device_plan), keep a row plan read back to the host (_RowPlan)
+and buffers of the labelled rows.  No row is ever permuted: the hidden states are read
 in place, the statistics need no unsort, and the backward forms the [M, H] gradient in one gather
 from the packed rows, scaled by the loss scale on the way.  The gradient is taken in the forward
 because the head is frozen.
 
 CHUNK_ROWS keeps the reference's name; its value is MI355X's: the reference's 256 rows bound
-the logits buffer on a 15 GB card (78 MB), while 2048 rows (622 MB, plus the labelled rows'
-gradient buffer, of 288 GB) let the two chunk GEMMs run at a size hipBLASLt handles efficiently
+the logits buffer on a 15 GB card (78 MB), while 2048 rows (622 MB, plus a gradient buffer of
+that size, of 288 GB) let the two chunk GEMMs run at a size hipBLASLt handles efficiently
 (the head's forward + backward at 2048 tokens: 2.2 ms against 4.6 ms in 256-row chunks).
-Every row's statistics and gradient are computed from that row alone, so no output depends on
-the chunking.
+Every row's statistics and gradient are computed from that row alone: on the chunking depends
+nothing but the order of dh's fp32 sums (the cut of the contraction follows from the rows).
 """
 
 import math
