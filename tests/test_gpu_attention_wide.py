@@ -4,13 +4,14 @@ outputs and log-sum-exps must be the same bits: the wide launch of many rows aga
 row, which is small enough for the 64-query kernel.  Row lengths: whole 128-query blocks, one query
 over, an odd 64-key block, shorter than one wavefront's 32 queries, empty (varlen)."""
 
+import ctypes
 import math
 
 import pytest
 import torch
 
 from tests.test_gpu_attention import reference
-from testt_amd import attention
+from testt_amd import _ext, attention
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
@@ -18,9 +19,12 @@ D, NH, NKV = 128, 12, 2
 SCALE = 1.0 / math.sqrt(D)
 
 
-def _wide(units, length):
+def _wide(varlen, rows, length):
+    """The forward's kernels for `rows` rows of T = length positions, or of length tokens in all."""
+    out = ctypes.c_int32(-1)
     cus = torch.cuda.get_device_properties(DEV).multi_processor_count
-    return units * -(-length // 128) * 4 >= 5 * cus
+    _ext.call("soupk_attention_wide", varlen, 0, rows, length, NH, cus, ctypes.addressof(out))
+    return out.value == 1
 
 
 LENGTHS = [256, 129, 193, 31, 128, 65, 255, 1] * 4
@@ -28,7 +32,7 @@ LENGTHS = [256, 129, 193, 31, 128, 65, 255, 1] * 4
 
 def test_padded_wide_matches_row_launches_and_fp32():
     B, T = len(LENGTHS), 256
-    assert _wide(B * NH, T) and not _wide(NH, T)
+    assert _wide(0, B, T) and not _wide(0, 1, T)
     g = torch.Generator().manual_seed(3)
     q = torch.randn(B, NH, T, D, generator=g).to(torch.float16)
     k = torch.randn(B, NKV, T, D, generator=g).to(torch.float16)
@@ -57,7 +61,7 @@ def test_padded_wide_matches_row_launches_and_fp32():
 @pytest.mark.parametrize("lengths", [LENGTHS, [700, 0, 130, 1, 515, 64] * 3])
 def test_varlen_wide_matches_row_launches(lengths):
     M, B = sum(lengths), len(lengths)
-    assert _wide(B * NH, M // B)
+    assert _wide(1, B, M)
     g = torch.Generator().manual_seed(M)
     rows = torch.randn(M, (NH + 2 * NKV) * D, generator=g).to(torch.float16).to(DEV)
     cu = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32,
@@ -69,7 +73,7 @@ def test_varlen_wide_matches_row_launches(lengths):
     for n in lengths:
         if n:
             one = torch.tensor([0, n], dtype=torch.int32, device=DEV)
-            assert not _wide(NH, n)
+            assert not _wide(1, 1, n)
             o1, l1 = attention.attention_varlen_fwd(rows[at:at + n].contiguous(), one, NH, NKV,
                                                     SCALE)
             assert torch.equal(o1.view(torch.int16), out[at:at + n].view(torch.int16)), n
