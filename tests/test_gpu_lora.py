@@ -248,6 +248,20 @@ def test_lora_row_counts(M):
 
 @pytest.mark.parametrize("M", [3071, 3072, 6144, 6401])
 def test_lora_bwd_params_slices(M):
-    """The last row count of 128-row slices, the first of 256- and of 512-row slices, and a last
-    slice of one row."""
+    """Many slices: a last one of 127 rows, whole ones, and a last slice of one row."""
     test_lora_bwd_params(M, 512, 512, 256, 2.0, True)
+
+
+@pytest.mark.parametrize("M", [300, 4096, 8192])
+def test_lora_bwd_params_sums_run_over_128_rows(M):
+    """128 terms of 1 in the second 128 rows, between terms of 2^30 and -2^30 in the first and the
+    last row: 128 is one fp32 ulp there, so the sum is kept exactly when those rows are added up
+    on their own first, and lost when one fp32 chain runs through the first 256 rows."""
+    H, NQ, NV = 256, 256, 128
+    x = torch.zeros(M, 1, dtype=torch.float16)
+    x[0], x[128:256], x[-1] = 32768.0, 1.0, -32768.0
+    z = x.abs()
+    y, g_q, g_v = (x.expand(M, n).contiguous().to(DEV) for n in (H, NQ, NV))
+    t = z.expand(M, 32).contiguous().to(DEV)
+    for d in lora.lora_bwd_params(y, t, t, g_q, g_v, 1.0):
+        assert torch.equal(d, torch.full_like(d, 128.0))

@@ -574,15 +574,18 @@ __global__ __launch_bounds__(kThreads) void lora_bwd_rows_kernel(
 //   dBq[j][i] = fp16(sum_m gs_q[m][j] t[m][i])        j < NQ, i < r,  gs_x = fp16(g_x * s)
 //   dBv[j][i] = fp16(sum_m gs_v[m][j] t[m][r + i])    j < NV, i < r
 // each cast to fp32 (the fp16 GEMM result cast to the fp32 parameter, as autocast's backward
-// gives it).  lora_params_partial_kernel: workgroup (column block of 64, slice of rows)
+// gives it).  lora_params_partial_kernel: workgroup (column block of 64, slice of kSlice rows)
 // stages 64-row chunks of X (y, or g_q / g_v scaled and rounded to gs as they are staged: its
 // 64 columns) and Z (dt or t) through LDS,
 // transposed so that each MFMA operand is 8 consecutive rows of one column, and writes fp32
 // partial sums per slice; lora_params_reduce_kernel adds the slices in order and rounds.
 // With the next chunk's loads issued before the current chunk's MFMAs and the reduce's loads
 // issued eight slices at a time, the pair took 10.5 us against 13.2 us at 2048 rows on
-// MI355X (identical bits).  The slices grow with the rows (params_slice).
-constexpr int kSlice = 128;        // rows of the smallest slice
+// MI355X (identical bits).  128 rows a slice at any row count, so that a long sequence's sums keep
+// short fp32 chains: slices that grow with the rows save writing and reading partial sums (128- /
+// 256- / 512-row slices: 888 rows 8.0 / 9.4 / 12.9 us, 2048 rows 10.9 / 10.4 / 13.7, 4096 rows
+// 16.2 / 13.8 / 15.6, 8192 rows 28.5 / 25.1 / 22.0), but lose small terms beside large ones.
+constexpr int kSlice = 128;        // rows per slice
 constexpr int kChunk = 64;         // rows per LDS chunk
 constexpr int kPStride = kChunk + 8;   // transposed tile row (halves): 144 B, 16-B aligned
 
@@ -617,7 +620,7 @@ __global__ __launch_bounds__(kThreads) void lora_params_partial_kernel(
     const uint16_t* __restrict__ y, const uint16_t* __restrict__ t,
     const uint16_t* __restrict__ dt, const uint16_t* __restrict__ gq, int64_t ldq,
     const uint16_t* __restrict__ gv, int64_t ldv, float scaling, float* __restrict__ part, int M,
-    int H, int NQ, int NV, int64_t n_out, int slice_rows) {
+    int H, int NQ, int NV, int64_t n_out) {
   __shared__ __align__(16) _Float16 XT[64 * kPStride];       // [64 columns][64 rows]
   __shared__ __align__(16) _Float16 ZT[2 * kR * kPStride];   // [32 columns][64 rows]
   const int nba = H / 64, nbq = NQ / 64;
@@ -631,7 +634,7 @@ __global__ __launch_bounds__(kThreads) void lora_params_partial_kernel(
   const uint16_t* Z = (kind == 0 ? dt : t) + (kind == 2 ? kR : 0);
   const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
   const int ql = lane & 15, gr = lane >> 4;
-  const int r_begin = slice * slice_rows, r_end = min(M, r_begin + slice_rows);
+  const int r_begin = slice * kSlice, r_end = min(M, r_begin + kSlice);
   // dA: C = X^T Z tiles (row = X column, column = Z column): wave w owns X columns 16w..+15
   //     and both Z tiles; dB: C = Z^T X (row = Z column, column = X column): wave w owns X
   //     columns 16w..+15.  Either way a lane's 4 results are 4 consecutive partial entries.
@@ -834,19 +837,6 @@ static int64_t lora_params_workspace(int64_t M, int32_t H, int32_t NQ, int32_t N
 
 namespace {
 
-// Rows per slice: kSlice while that gives at most two dozen slices, then the power of two that leaves
-// 12 to 24 of them, so that the partial sums (312 KB a slice) written and read back stop growing
-// with the rows.  From 3072 rows on an fp32 sum thus runs over 256 or more rows instead of 128 before
-// the slices are added; the gradients are rounded to fp16 after that, and their error against 64
-// bits is the same (2 x 4096 tokens: 2.6e-3 either way).  Measured with 128- / 256- / 512-row slices: 888 rows 8.0 / 9.4 /
-// 12.9 us, 2048 rows 10.9 / 10.4 / 13.7, 4096 rows 16.2 / 13.8 / 15.6, 8192 rows 28.5 / 25.1 /
-// 22.0.
-int params_slice(int64_t M) {
-  int64_t rows = kSlice;
-  while (M / (2 * rows) >= 12) rows *= 2;
-  return static_cast<int>(rows);
-}
-
 // The two launches of the parameter gradients over a caller-given partial-sum buffer `part`
 // (at least lora_params_workspace(M, H, NQ, NV) floats).  The partial kernel writes every
 // entry of every slice, so `part` needs no clearing and its old contents never leak into a
@@ -862,12 +852,11 @@ int lora_params_launch(const uint16_t* y, const uint16_t* t, const uint16_t* dt,
     return launch_kernel(lora_params_reduce_kernel, dim3(reduce_grid), dim3(256), st,
                          static_cast<const float*>(nullptr), 0, n_out, H, NQ, d_aq, d_av,
                          d_bq, d_bv);
-  const int slice_rows = params_slice(M);
-  const int slices = static_cast<int>((M + slice_rows - 1) / slice_rows);
+  const int slices = static_cast<int>((M + kSlice - 1) / kSlice);
   const dim3 grid(static_cast<unsigned>(H / 64 + NQ / 64 + NV / 64),
                   static_cast<unsigned>(slices));
   int rc2 = launch_kernel(lora_params_partial_kernel, grid, dim3(kThreads), st, y, t, dt, g_q,
-                          ld_q, g_v, ld_v, scaling, part, static_cast<int>(M), H, NQ, NV, n_out, slice_rows);
+                          ld_q, g_v, ld_v, scaling, part, static_cast<int>(M), H, NQ, NV, n_out);
   if (rc2 != kOk) return rc2;
   return launch_kernel(lora_params_reduce_kernel, dim3(reduce_grid), dim3(256), st, part,
                        slices, n_out, H, NQ, d_aq, d_av, d_bq, d_bv);
