@@ -469,10 +469,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_fwd_kernel(AttnParams p) {
 // long as its MFMAs (each 1024 clocks per CU), here half as long.  The next block's tiles go from
 // registers into the other of two LDS buffers, one barrier per block, and two workgroups fit a
 // CU (73.9 KB of LDS, two wavefronts per SIMD), so one's softmax runs under the other's MFMAs.
-// 2 x 4096 tokens, 12 heads: 222 -> 141 us (464 -> 733 TFLOP/s).  What is left is the chain of a
+// 2 x 4096 tokens, 12 heads: 215 -> 134 us (480 -> 770 TFLOP/s).  What is left is the chain of a
 // block (scores, maxima, exponentials, products) at two wavefronts per SIMD: by the counters 28 LDS
 // instructions for a 16-query tile's block instead of 58, and no unit near its limit (matrix cores
-// busy 31%, vector ALU 38%, LDS 32%, 1.94 wavefronts per SIMD).  A workgroup order that
+// busy 31%, vector ALU 41%, LDS 32%, 1.94 wavefronts per SIMD).  A workgroup order that
 // gives each XCD's L2 its own heads measured nothing on even rows and 129 -> 251 us on rows of 4096
 // to 1024 tokens (the XCDs' shares differ); raising the wave priority around the MFMAs 150 -> 157 us.
 constexpr int kWideBQ = 128;
